@@ -1,0 +1,15 @@
+// Instantiations of matmul_tile for Q5_0 and Q5_1 (units of their own so that the formats compile in parallel).
+#include "matmul_tile.hpp"
+
+namespace slhip {
+
+int launch_tile_part3(int fmt, const MatvecArgs& a, bool dual, hipStream_t st)
+{
+    switch (fmt) {
+    case SLHIP_FMT_Q5_0: return launch_tile_fmt<SLHIP_FMT_Q5_0>(a, dual, st);
+    case SLHIP_FMT_Q5_1: return launch_tile_fmt<SLHIP_FMT_Q5_1>(a, dual, st);
+    default: return SLHIP_ERR_UNSUPPORTED;
+    }
+}
+
+}  // namespace slhip

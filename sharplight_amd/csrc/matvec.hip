@@ -626,139 +626,10 @@ __global__ __launch_bounds__(kMqThreads) void matvec_quant(MatvecArgs a)
 // split into three bf16 parts h + m + l = x exactly (each part the round-to-nearest-even of the remainder;
 // f32 has 24 significant bits, bf16 8), so every product w * part is exact and the sums stay f32: the
 // result has the error of f32 accumulation, like the VALU kernel. bf16 x is one part. A block of 8 waves
-// takes a 16-row tile (pair); the waves split K, each lane loading 2 x 16 bytes per row per 64 values (two
-// instructions covering 64 contiguous bytes of 16 rows each); partial tiles meet in LDS.
+// takes a 16-row tile (pair); the waves split K; partial tiles meet in LDS.
 constexpr int kMmWaves = 8;
 
-template <bool DUAL, bool XF32>
-__global__ __launch_bounds__(64 * kMmWaves) void matvec_mfma(MatvecArgs a)
-{
-    __shared__ f32x4_t red[kMmWaves][2][64];
-    const int lane = threadIdx.x & 63;
-    const int wave = wave_id();
-    const int r = lane & 15, g = lane >> 4;
-    const int64_t n0 = static_cast<int64_t>(blockIdx.x) * 16;
-    const int64_t row = n0 + r < a.N ? n0 + r : a.N - 1;
-    int64_t tok = a.t0 + r;
-    tok = tok < a.T ? tok : a.T - 1;
-    const int nc = static_cast<int>(a.K / 64);
-    const int c0 = wave * nc / kMmWaves, c1 = (wave + 1) * nc / kMmWaves;
-    const char* wg = a.wg + row * a.wrow;
-    const char* wu = DUAL ? a.wu + row * a.wrow : nullptr;
-    f32x4_t ag = {0.0f, 0.0f, 0.0f, 0.0f}, au = {0.0f, 0.0f, 0.0f, 0.0f};
-    // One chunk's operands as loaded: weights (gate, up: two 16-byte vectors each) and x (f32: four float4;
-    // bf16: two uint4 in xb). The next chunk's loads are issued before the current chunk is computed.
-    struct Ops {
-        uint4 A0, A1, U0, U1;
-        float4 xf[4];
-        uint4 xb[2];
-    };
-    auto load = [&](int c, Ops& o) {
-        const int64_t k0 = static_cast<int64_t>(c) * 64 + 8 * g;  // step 0: 64c + 8g + j; step 1: + 32
-        o.A0 = load_nt(wg + k0 * 2);
-        o.A1 = load_nt(wg + (k0 + 32) * 2);
-        if (DUAL) {
-            o.U0 = load_nt(wu + k0 * 2);
-            o.U1 = load_nt(wu + (k0 + 32) * 2);
-        }
-        if (XF32) {
-            const float* xr = static_cast<const float*>(a.x) + tok * a.xs + k0;
-            o.xf[0] = *reinterpret_cast<const float4*>(xr);
-            o.xf[1] = *reinterpret_cast<const float4*>(xr + 4);
-            o.xf[2] = *reinterpret_cast<const float4*>(xr + 32);
-            o.xf[3] = *reinterpret_cast<const float4*>(xr + 36);
-        } else {
-            const uint16_t* xr = static_cast<const uint16_t*>(a.x) + tok * a.xs + k0;
-            o.xb[0] = *reinterpret_cast<const uint4*>(xr);
-            o.xb[1] = *reinterpret_cast<const uint4*>(xr + 32);
-        }
-    };
-    auto compute = [&](const Ops& o) {
-        uint4 B[2][3];
-        int np = 1;
-        if (XF32) {
-#pragma unroll
-            for (int s2 = 0; s2 < 2; s2++) {
-                const float4 f0 = o.xf[2 * s2], f1 = o.xf[2 * s2 + 1];
-                const float xv[8] = {f0.x, f0.y, f0.z, f0.w, f1.x, f1.y, f1.z, f1.w};
-                split3(xv, B[s2][0], B[s2][1], B[s2][2]);
-            }
-            np = 3;
-        } else {
-            B[0][0] = o.xb[0];
-            B[1][0] = o.xb[1];
-        }
-#pragma unroll
-        for (int p = 0; p < 3; p++) {
-            if (p >= np) break;
-            ag = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(o.A0), as_bf16x8(B[0][p]), ag, 0, 0, 0);
-            ag = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(o.A1), as_bf16x8(B[1][p]), ag, 0, 0, 0);
-            if (DUAL) {
-                au = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(o.U0), as_bf16x8(B[0][p]), au, 0, 0, 0);
-                au = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(o.U1), as_bf16x8(B[1][p]), au, 0, 0, 0);
-            }
-        }
-    };
-    // Two operand sets in alternation (a copy between them would wait for the loads): each chunk's loads are
-    // issued before the previous chunk is computed. The scheduling barriers keep them there -- left free, the
-    // scheduler sinks the loads below the MFMAs and every chunk waits for its own loads.
-    const int n = c1 - c0;
-    if (n > 0) {  // wave-uniform
-        Ops oa, ob;
-        load(c0, oa);
-        int i = 0;
-        for (; i + 2 < n; i += 2) {  // branch-free body: a merge would make the load counter waits exact-zero
-            load(c0 + i + 1, ob);
-            __builtin_amdgcn_sched_barrier(0);
-            compute(oa);
-            __builtin_amdgcn_sched_barrier(0);
-            load(c0 + i + 2, oa);
-            __builtin_amdgcn_sched_barrier(0);
-            compute(ob);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        if (i + 1 < n) {  // two chunks left
-            load(c0 + i + 1, ob);
-            __builtin_amdgcn_sched_barrier(0);
-            compute(oa);
-            __builtin_amdgcn_sched_barrier(0);
-            compute(ob);
-        } else {
-            compute(oa);
-        }
-    }
-    red[wave][0][lane] = ag;
-    if (DUAL) red[wave][1][lane] = au;
-    __syncthreads();
-    if (wave != 0) return;
-#pragma unroll
-    for (int w = 1; w < kMmWaves; w++) {
-        ag += red[w][0][lane];
-        if (DUAL) au += red[w][1][lane];
-    }
-    // lane: token column r, rows 4g + i
-    const int64_t t = a.t0 + r;
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const int64_t n = n0 + 4 * g + i;
-        float out = ag[i];
-        if (DUAL) {
-            const float act = a.act == SLHIP_ACT_SILU        ? activate<SLHIP_ACT_SILU>(ag[i])
-                              : a.act == SLHIP_ACT_GELU_TANH ? activate<SLHIP_ACT_GELU_TANH>(ag[i])
-                                                             : activate<SLHIP_ACT_GELU_ERF>(ag[i]);
-            out = act * au[i];
-        }
-        if (t < a.T && n < a.N) {
-            if (!DUAL && a.bias) out = out + a.bias[n];
-            if (a.yt == SLHIP_F32)
-                static_cast<float*>(a.y)[t * a.ys + n] = out;
-            else
-                static_cast<uint16_t*>(a.y)[t * a.ys + n] = static_cast<uint16_t>(f32_to_bf16_bits(out));
-        }
-    }
-}
-
-// The same product with the weights staged row by row: reading a 16-row tile straight into MFMA operands
+// The weights are staged row by row: reading a 16-row tile straight into MFMA operands
 // puts 16 rows x 64 bytes in every load instruction, a pattern HBM serves at ~5.0 TB/s, while 1 KiB of one
 // or two rows per instruction streams at ~6.4 TB/s. So per stage of SK values, the block loads the tile's
 // rows contiguously into LDS (row pitch SK*2 + 16 bytes: the 16 rows of an A fragment fall 4 banks apart),
@@ -905,371 +776,6 @@ __global__ __launch_bounds__(64 * kMmWaves) void matvec_mfma_lds(MatvecArgs a)
 #pragma unroll
     for (int i = 0; i < 4; i++) {
         const int64_t n = n0 + 16 * tt + 4 * g + i;
-        float out = sg[i];
-        if (DUAL) {
-            const float act = a.act == SLHIP_ACT_SILU        ? activate<SLHIP_ACT_SILU>(sg[i])
-                              : a.act == SLHIP_ACT_GELU_TANH ? activate<SLHIP_ACT_GELU_TANH>(sg[i])
-                                                             : activate<SLHIP_ACT_GELU_ERF>(sg[i]);
-            out = act * su[i];
-        }
-        if (t < a.T && n < a.N) {
-            if (!DUAL && a.bias) out = out + a.bias[n];
-            if (a.yt == SLHIP_F32)
-                static_cast<float*>(a.y)[t * a.ys + n] = out;
-            else
-                static_cast<uint16_t*>(a.y)[t * a.ys + n] = static_cast<uint16_t>(f32_to_bf16_bits(out));
-        }
-    }
-}
-
-// ---- block formats at several tokens on the matrix cores -------------------------------------------------
-//
-// The VALU kernel decodes every weight once per group of tokens, so its time grows with T (Q4_0 dual at
-// [14336, 4096]: 18 us at T = 1, 57 at 4, 218 at 16). Here a 16-row tile's blocks are staged raw in LDS and
-// each code is decoded once into a bf16 A fragment that serves all 16 token columns of
-// v_mfma_f32_16x16x32_bf16: a 32-value block is one MFMA k-step, so each block's sums (16 rows x 16 tokens)
-// come out of one short MFMA chain and take the block scale d on the VALU (acc += d * sum). The codes enter
-// exactly (Q4_0: q - 8, Q8_0: q; small integers are exact in bf16); f32 x enters as two bf16 parts h + m
-// (h = bf16(x), m = bf16(x - h): |x - h - m| <= 2^-18 |x|, inside the matvec bound), bf16 x as it is. Q4_K
-// takes the same path with its 32-value sub-blocks as the blocks (a stage is 4 super-blocks, 576 bytes of a
-// row, and a wave half a super-block): codes q enter as they are, and the sub-block's d0 = d sc and minimum
-// m = dmin mn are applied on the VALU as acc += d0 sum(q x) - m sum(x), sum(x) of the lane's token summed
-// across its four lane groups (Quant.cs:518-545's value d0 q - m). Q6_K too (a stage is 2 super-blocks, 420
-// bytes staged with 4-byte loads, and a wave a quarter super-block): codes enter as q - 32, and since a
-// 32-value block holds two 16-value scale groups, each block takes two MFMA chains, lane groups 0-1 (the
-// first group's values) in one and 2-3 in the other, the other half's codes masked to zero. The other block
-// formats follow the same pattern: Q4_1 and Q5_1 add m sum(x) per block, Q5_0 and Q5_1 take the 17th code
-// bit from their qh word, Q5_K is Q4_K with qh bit j of byte l, and Q2_K / Q3_K (16-value scale groups, as
-// Q6_K; Q3_K's codes q + 4h - 4, Q2_K's per-half minimum dmin m sum(x) over each half). A block of 8 waves
-// takes one tile; the waves split each stage's blocks; the stage's row bytes are loaded two stages
-// ahead into registers and written to LDS one stage ahead (as the bf16 kernel above); partial sums meet in
-// LDS at the end.
-__device__ __forceinline__ void q4k_scales(const uint4& hdr, int j, float& d0, float& m);  // defined below
-
-template <int FMT, bool DUAL, bool XF32>
-__global__ __launch_bounds__(64 * kMqWaves) void matvec_mfma_q(MatvecArgs a)
-{
-    constexpr int BB = Fmt<FMT>::BB;
-    constexpr int NM = DUAL ? 2 : 1;
-    constexpr int SKB = MqGeom<FMT>::SKB;
-    constexpr bool KQ = FMT == SLHIP_FMT_Q4_K || FMT == SLHIP_FMT_Q5_K;  // 8 sub-blocks, d0 q - m
-    constexpr bool Q2K = FMT == SLHIP_FMT_Q2_K, Q3K = FMT == SLHIP_FMT_Q3_K;
-    constexpr bool K6 = FMT == SLHIP_FMT_Q6_K || Q2K || Q3K;  // two 16-value scale groups per 32-value block
-    constexpr bool MB = Fmt<FMT>::M && !Fmt<FMT>::K;  // Q4_1, Q5_1: d q + m per 32-value block
-    constexpr int SBB = Fmt<FMT>::BB;                  // K-quant super-block bytes
-    constexpr int RB = MqGeom<FMT>::RB;  // bytes of one row per stage
-    constexpr int UB = MqGeom<FMT>::UB;  // bytes per staging load
-    using WU = std::conditional_t<UB == 16, uint4, std::conditional_t<UB == 8, uint2, uint32_t>>;
-    constexpr int PITCH = RB + 16;
-    constexpr int UPR = RB / UB;  // staging units of a row per stage
-    constexpr int UNITS = NM * 16 * UPR;
-    constexpr int UPL = (UNITS + 64 * kMqWaves - 1) / (64 * kMqWaves);
-    constexpr int BPW = SKB / kMqWaves;  // blocks per wave and stage
-    static_assert(RB % UB == 0 && PITCH % UB == 0 && SKB % kMqWaves == 0, "stage shape");
-    static_assert(!(KQ || K6) || 8 % BPW == 0, "a K-quant wave takes whole blocks of one super-block");
-    static_assert(!KQ || BPW == 4, "a Q4_K wave takes the four sub-blocks of one packed scale word");
-    __shared__ __align__(16) uint8_t stage[2][NM][16][PITCH];
-    const int lane = threadIdx.x & 63;
-    const int wave = wave_id();
-    const int r = lane & 15, g = lane >> 4;
-    const int64_t n0 = static_cast<int64_t>(blockIdx.x) * 16;
-    int64_t tok = a.t0 + r;
-    tok = tok < a.T ? tok : a.T - 1;
-    const int ns = static_cast<int>(a.K / (SKB * 32));  // stages (each SKB * 32 values of the row)
-
-    // this thread's 16-byte units of the stage (threads past the last unit repeat it)
-    const char* src[UPL];
-    int dst[UPL];
-#pragma unroll
-    for (int i = 0; i < UPL; i++) {
-        int u = static_cast<int>(threadIdx.x) + 64 * kMqWaves * i;
-        u = u < UNITS ? u : UNITS - 1;
-        const int m = u / (16 * UPR), rem = u - m * (16 * UPR), rr = rem / UPR, c = rem - rr * UPR;
-        int64_t row = n0 + rr;
-        row = row < a.N ? row : a.N - 1;
-        src[i] = (m == 0 ? a.wg : a.wu) + row * a.wrow + UB * c;
-        dst[i] = (m * 16 + rr) * PITCH + UB * c;
-    }
-    WU pa[UPL], pb[UPL];
-    auto fetch_w = [&](WU* pw, int s) {
-#pragma unroll
-        for (int i = 0; i < UPL; i++) {
-            const char* p = src[i] + static_cast<int64_t>(s) * RB;
-            if constexpr (UB == 16) {
-                pw[i] = load_nt(p);
-            } else if constexpr (UB == 8) {
-                const u32x2 v = __builtin_nontemporal_load(reinterpret_cast<const u32x2*>(p));
-                pw[i] = make_uint2(v.x, v.y);
-            } else {
-                pw[i] = __builtin_nontemporal_load(reinterpret_cast<const uint32_t*>(p));
-            }
-        }
-    };
-    auto put_w = [&](const WU* pw, int b) {
-#pragma unroll
-        for (int i = 0; i < UPL; i++) *reinterpret_cast<WU*>(&stage[b][0][0][0] + dst[i]) = pw[i];
-    };
-    // x of the wave's blocks, one stage ahead in two register sets: lane (g, token r) holds values 8g .. 8g + 7
-    struct Xs {
-        float4 f[BPW][2];
-        uint4 b[BPW];
-    };
-    auto fetch_x = [&](Xs& x, int s) {
-#pragma unroll
-        for (int j = 0; j < BPW; j++) {
-            const int64_t k0 = (static_cast<int64_t>(s) * SKB + wave * BPW + j) * 32 + 8 * g;
-            if (XF32) {
-                const float* xr = static_cast<const float*>(a.x) + tok * a.xs + k0;
-                x.f[j][0] = *reinterpret_cast<const float4*>(xr);
-                x.f[j][1] = *reinterpret_cast<const float4*>(xr + 4);
-            } else {
-                x.b[j] = *reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(a.x) + tok * a.xs + k0);
-            }
-        }
-    };
-    f32x4_t ag = {0.0f, 0.0f, 0.0f, 0.0f}, au = {0.0f, 0.0f, 0.0f, 0.0f};
-    // Stage s from LDS buffer s & 1 with x in xc; the next stage's x (into xn) and the weights two ahead go
-    // out first, then each block in turn: its codes and scales from LDS, x split, the MFMAs, the scaling.
-    auto run_stage = [&](int s, const Xs& xc, Xs& xn, WU* wnext, WU* wfree) {
-        const int b = s & 1;
-        if (s + 1 < ns) fetch_x(xn, s + 1);  // block-uniform conditions
-        if (s + 2 < ns) fetch_w(wfree, s + 2);
-        __builtin_amdgcn_sched_barrier(0);
-        // Q4_K: the wave's half super-block (sub-blocks 4 (wave & 1) ..); the headers of the rows its sums
-        // belong to (4g .. 4g + 3) are read once per stage. (Decoding the (d0, m) pairs once per wave into an
-        // LDS table instead cost a block of residency per CU: 82 -> 116 us at 16 tokens.)
-        // K-quants: the wave's blocks u0 .. u0 + BPW - 1 of the stage's super-block (wave BPW) / 8
-        const int u0 = (wave * BPW) & 7;
-        const int sbo = (KQ || K6) ? ((wave * BPW) >> 3) * SBB : 0;
-        // Q4_K: per row 4g + i its d, dmin and the packed 6-bit scales and minima of the wave's four sub-blocks
-        // (byte j of scw / mnw: sub-block u0 + j; Quant.cs:518-545's packing), so that a sub-block's d0 and m
-        // are one byte conversion and one multiply each
-        float kdg[4], kmg[4], kdu[4], kmu[4];
-        uint32_t scg[4], mng[4], scu[4], mnu[4];
-        // Q6_K / Q3_K / Q2_K: the super-block scale d (Q2_K: and dmin) of the rows 4g + i
-        float d6g[4], d6u[4], n6g[4], n6u[4];
-        if constexpr (K6) {
-            constexpr int DO = Q2K ? 80 : Q3K ? 108 : 208;
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                d6g[i] = static_cast<float>(*reinterpret_cast<const _Float16*>(&stage[b][0][4 * g + i][sbo + DO]));
-                d6u[i] = DUAL ? static_cast<float>(*reinterpret_cast<const _Float16*>(&stage[b][NM - 1][4 * g + i][sbo + DO]))
-                              : 0.0f;
-                if constexpr (Q2K) {
-                    n6g[i] = static_cast<float>(*reinterpret_cast<const _Float16*>(&stage[b][0][4 * g + i][sbo + 82]));
-                    n6u[i] = DUAL ? static_cast<float>(*reinterpret_cast<const _Float16*>(&stage[b][NM - 1][4 * g + i][sbo + 82]))
-                                  : 0.0f;
-                }
-            }
-        }
-        if constexpr (KQ) {
-            auto words = [&](const uint4& h, float& d, float& dm, uint32_t& sc, uint32_t& mn) {
-                d = f16_lo(h.x);
-                dm = f16_hi(h.x);
-                if (u0 < 4) {  // sub-blocks 0-3: the low 6 bits of bytes 4..7 (scales) and 8..11 (minima)
-                    sc = h.y & 0x3F3F3F3Fu;
-                    mn = h.z & 0x3F3F3F3Fu;
-                } else {  // 4-7: low / high nibbles of bytes 12..15, top two bits of bytes 4..11
-                    sc = (h.w & 0x0F0F0F0Fu) | ((h.y >> 2) & 0x30303030u);
-                    mn = ((h.w >> 4) & 0x0F0F0F0Fu) | ((h.z >> 2) & 0x30303030u);
-                }
-            };
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                words(*reinterpret_cast<const uint4*>(&stage[b][0][4 * g + i][sbo]), kdg[i], kmg[i], scg[i], mng[i]);
-                if (DUAL)
-                    words(*reinterpret_cast<const uint4*>(&stage[b][NM - 1][4 * g + i][sbo]), kdu[i], kmu[i], scu[i], mnu[i]);
-            }
-        }
-#pragma unroll
-        for (int j = 0; j < BPW; j++) {
-            const int off = (wave * BPW + j) * BB;
-            const int sj = u0 + j;  // K-quant 32-value block (0..7) in its super-block
-            uint4 Ag, Au;
-            if constexpr (KQ) {
-                constexpr bool FIVE = FMT == SLHIP_FMT_Q5_K;
-                Ag = q4k_codes<FIVE>(&stage[b][0][r][0], sbo, sj, g);
-                Au = DUAL ? q4k_codes<FIVE>(&stage[b][NM - 1][r][0], sbo, sj, g) : Ag;
-            } else if constexpr (Q2K || Q3K) {
-                Ag = q23k_codes<Q3K>(&stage[b][0][r][0], sbo, sj, g);
-                Au = DUAL ? q23k_codes<Q3K>(&stage[b][NM - 1][r][0], sbo, sj, g) : Ag;
-            } else if constexpr (K6) {
-                Ag = q6k_codes(&stage[b][0][r][0], sbo, sj, g);
-                Au = DUAL ? q6k_codes(&stage[b][NM - 1][r][0], sbo, sj, g) : Ag;
-            } else {
-                Ag = mq_codes<FMT>(&stage[b][0][r][0], off, g);
-                Au = DUAL ? mq_codes<FMT>(&stage[b][NM - 1][r][0], off, g) : Ag;
-            }
-            float dg[4], du[4], mg[4], mu[4];
-            float ng0[4], ng1[4], nu0[4], nu1[4];  // Q2_K: the two halves' minima dmin * m
-#pragma unroll
-            for (int i = 0; i < 4; i++) {  // the scales of the rows this lane's sums belong to (4g .. 4g + 3)
-                if constexpr (Q2K) {
-                    // scale bytes 8n + 2j + 0..1 (the block's two halves): d (low nibble), dmin (high nibble)
-                    auto sc2 = [&](const uint8_t* row, float d, float dm, float& s0, float& s1, float& m0, float& m1) {
-                        const uint32_t v = *reinterpret_cast<const uint16_t*>(row + sbo + 2 * sj);
-                        s0 = __fmul_rn(d, static_cast<float>(v & 0xFu));
-                        s1 = __fmul_rn(d, static_cast<float>((v >> 8) & 0xFu));
-                        m0 = __fmul_rn(dm, static_cast<float>((v >> 4) & 0xFu));
-                        m1 = __fmul_rn(dm, static_cast<float>(v >> 12));
-                    };
-                    sc2(&stage[b][0][4 * g + i][0], d6g[i], n6g[i], dg[i], mg[i], ng0[i], ng1[i]);
-                    if (DUAL) sc2(&stage[b][NM - 1][4 * g + i][0], d6u[i], n6u[i], du[i], mu[i], nu0[i], nu1[i]);
-                } else if constexpr (Q3K) {
-                    // 6-bit scales s = 8n + 2j + 0..1: low 4 bits from bytes 96 + 4 (w & 1) + b (the low nibble
-                    // for w < 2), high 2 from bits 2w of bytes 104 + b, w = s / 4, b = s % 4; d (s - 32)
-                    const int s0 = 2 * sj, w = s0 >> 2, b0 = s0 & 3;
-                    auto sc3 = [&](const uint8_t* row, float d, float& o0, float& o1) {
-                        const uint32_t a = *reinterpret_cast<const uint16_t*>(row + sbo + 96 + 4 * (w & 1) + b0);
-                        const uint32_t h = *reinterpret_cast<const uint16_t*>(row + sbo + 104 + b0);
-                        const uint32_t lo = w < 2 ? (a & 0x0F0Fu) : ((a >> 4) & 0x0F0Fu);
-                        const uint32_t sc = lo | (((h >> (2 * w)) & 0x0303u) << 4);
-                        o0 = __fmul_rn(d, static_cast<float>(static_cast<int>(sc & 0xFFu) - 32));
-                        o1 = __fmul_rn(d, static_cast<float>(static_cast<int>(sc >> 8) - 32));
-                    };
-                    sc3(&stage[b][0][4 * g + i][0], d6g[i], dg[i], mg[i]);
-                    if (DUAL) sc3(&stage[b][NM - 1][4 * g + i][0], d6u[i], du[i], mu[i]);
-                } else if constexpr (KQ) {
-                    const uint32_t sh = 8 * static_cast<uint32_t>(j);  // byte j: sub-block u0 + j
-                    dg[i] = __fmul_rn(kdg[i], static_cast<float>((scg[i] >> sh) & 0xFFu));
-                    mg[i] = __fmul_rn(kmg[i], static_cast<float>((mng[i] >> sh) & 0xFFu));
-                    if (DUAL) {
-                        du[i] = __fmul_rn(kdu[i], static_cast<float>((scu[i] >> sh) & 0xFFu));
-                        mu[i] = __fmul_rn(kmu[i], static_cast<float>((mnu[i] >> sh) & 0xFFu));
-                    }
-                } else if constexpr (K6) {
-                    // the block's two 16-value scales sc[8 hf + 2k + 0..1] (2-byte aligned): d sc as (dg, mg)
-                    const int so = sbo + 192 + 2 * sj;
-                    const uint32_t sg = *reinterpret_cast<const uint16_t*>(&stage[b][0][4 * g + i][so]);
-                    dg[i] = __fmul_rn(d6g[i], static_cast<float>(static_cast<int8_t>(sg & 0xFFu)));
-                    mg[i] = __fmul_rn(d6g[i], static_cast<float>(static_cast<int8_t>(sg >> 8)));
-                    if (DUAL) {
-                        const uint32_t su = *reinterpret_cast<const uint16_t*>(&stage[b][NM - 1][4 * g + i][so]);
-                        du[i] = __fmul_rn(d6u[i], static_cast<float>(static_cast<int8_t>(su & 0xFFu)));
-                        mu[i] = __fmul_rn(d6u[i], static_cast<float>(static_cast<int8_t>(su >> 8)));
-                    }
-                } else {
-                    dg[i] = static_cast<float>(*reinterpret_cast<const _Float16*>(&stage[b][0][4 * g + i][off]));
-                    du[i] = DUAL ? static_cast<float>(*reinterpret_cast<const _Float16*>(&stage[b][NM - 1][4 * g + i][off]))
-                                 : 0.0f;
-                    if constexpr (MB) {  // the block minimum m (f16 after d)
-                        mg[i] = static_cast<float>(*reinterpret_cast<const _Float16*>(&stage[b][0][4 * g + i][off + 2]));
-                        mu[i] = DUAL ? static_cast<float>(*reinterpret_cast<const _Float16*>(&stage[b][NM - 1][4 * g + i][off + 2]))
-                                     : 0.0f;
-                    }
-                }
-            }
-            uint4 Bh, Bm;
-            float xsum = 0.0f;  // Q4_K: the sub-block's x sum of this lane's token (the min term)
-            if (XF32) {
-                const float v[8] = {xc.f[j][0].x, xc.f[j][0].y, xc.f[j][0].z, xc.f[j][0].w,
-                                    xc.f[j][1].x, xc.f[j][1].y, xc.f[j][1].z, xc.f[j][1].w};
-                split2(v, Bh, Bm);
-                if constexpr (KQ || MB || Q2K) xsum = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
-            } else {
-                Bh = xc.b[j];
-                if constexpr (KQ || MB || Q2K) {
-                    const uint4& w = xc.b[j];
-                    xsum = ((bf16_lo(w.x) + bf16_hi(w.x)) + (bf16_lo(w.y) + bf16_hi(w.y))) +
-                           ((bf16_lo(w.z) + bf16_hi(w.z)) + (bf16_lo(w.w) + bf16_hi(w.w)));
-                }
-            }
-            if constexpr (KQ || MB) {  // the four lane groups of the token hold the block's four 8-value parts
-                xsum += __shfl_xor(xsum, 16);
-                xsum += __shfl_xor(xsum, 32);
-            }
-            float xh0 = 0.0f, xh1 = 0.0f;  // Q2_K: the token's x sums over the block's two 16-value halves
-            if constexpr (Q2K) {
-                const float p01 = xsum + __shfl_xor(xsum, 16);  // lane groups {0, 1} or {2, 3}
-                const float other = __shfl_xor(p01, 32);
-                xh0 = g < 2 ? p01 : other;
-                xh1 = g < 2 ? other : p01;
-            }
-            if constexpr (K6) {
-                // Q6_K, Q3_K, Q2_K: lane groups 0-1 hold the block's first 16 values (scale dg), 2-3 the second (scale mg):
-                // one MFMA chain per half, the other half's codes masked to zero (a mask, not a select of
-                // vectors, which the compiler would lower to a stack array)
-                const uint32_t keep = g < 2 ? ~0u : 0u;
-                auto half = [&](const uint4& A, uint32_t k) { return make_uint4(A.x & k, A.y & k, A.z & k, A.w & k); };
-                const f32x4_t zero = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-                for (int m = 0; m < NM; m++) {
-                    const uint4& A = m == 0 ? Ag : Au;
-                    const uint4 A0 = half(A, keep), A1 = half(A, ~keep);
-                    f32x4_t c0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(A0), as_bf16x8(Bh), zero, 0, 0, 0);
-                    f32x4_t c1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(A1), as_bf16x8(Bh), zero, 0, 0, 0);
-                    if (XF32) {
-                        c0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(A0), as_bf16x8(Bm), c0, 0, 0, 0);
-                        c1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(A1), as_bf16x8(Bm), c1, 0, 0, 0);
-                    }
-                    f32x4_t& acc = m == 0 ? ag : au;
-                    const float* s0 = m == 0 ? dg : du;
-                    const float* s1 = m == 0 ? mg : mu;
-#pragma unroll
-                    for (int i = 0; i < 4; i++) acc[i] = fmaf(s1[i], c1[i], fmaf(s0[i], c0[i], acc[i]));
-                    if constexpr (Q2K) {  // - dmin m per half times the half's x sum
-                        const float* n0 = m == 0 ? ng0 : nu0;
-                        const float* n1 = m == 0 ? ng1 : nu1;
-#pragma unroll
-                        for (int i = 0; i < 4; i++) acc[i] = fmaf(-n1[i], xh1, fmaf(-n0[i], xh0, acc[i]));
-                    }
-                }
-                continue;
-            }
-            f32x4_t cg = {0.0f, 0.0f, 0.0f, 0.0f}, cu = {0.0f, 0.0f, 0.0f, 0.0f};
-            cg = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(Ag), as_bf16x8(Bh), cg, 0, 0, 0);
-            if (XF32) cg = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(Ag), as_bf16x8(Bm), cg, 0, 0, 0);
-            if (DUAL) {
-                cu = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(Au), as_bf16x8(Bh), cu, 0, 0, 0);
-                if (XF32) cu = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(Au), as_bf16x8(Bm), cu, 0, 0, 0);
-            }
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                ag[i] = fmaf(dg[i], cg[i], ag[i]);
-                if (DUAL) au[i] = fmaf(du[i], cu[i], au[i]);
-                if constexpr (KQ) {  // Q4_K, Q5_K: d0 sum(q x) - m sum(x)
-                    ag[i] = fmaf(-mg[i], xsum, ag[i]);
-                    if (DUAL) au[i] = fmaf(-mu[i], xsum, au[i]);
-                }
-                if constexpr (MB) {  // Q4_1, Q5_1: d sum(q x) + m sum(x)
-                    ag[i] = fmaf(mg[i], xsum, ag[i]);
-                    if (DUAL) au[i] = fmaf(mu[i], xsum, au[i]);
-                }
-            }
-        }
-        if (s + 1 < ns) put_w(wnext, b ^ 1);
-        __syncthreads();
-    };
-    Xs xa, xb;
-    fetch_x(xa, 0);
-    fetch_w(pa, 0);
-    if (ns > 1) fetch_w(pb, 1);
-    put_w(pa, 0);
-    __syncthreads();
-    int s = 0;
-    for (; s + 1 < ns; s += 2) {
-        run_stage(s, xa, xb, pb, pa);
-        run_stage(s + 1, xb, xa, pa, pb);
-    }
-    if (s < ns) run_stage(s, xa, xb, pb, pa);
-    // the waves' partial sums meet in the (now idle) stage memory: [wave][matrix][lane]
-    f32x4_t* red = reinterpret_cast<f32x4_t*>(&stage[0][0][0][0]);
-    static_assert(sizeof(stage) >= sizeof(f32x4_t) * kMqWaves * NM * 64, "reduction space");
-    red[(wave * NM) * 64 + lane] = ag;
-    if (DUAL) red[(wave * NM + 1) * 64 + lane] = au;
-    __syncthreads();
-    if (wave != 0) return;
-    f32x4_t sg = red[lane], su = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-    if (DUAL) su = red[64 + lane];
-#pragma unroll
-    for (int w = 1; w < kMqWaves; w++) {
-        sg += red[(w * NM) * 64 + lane];
-        if (DUAL) su += red[(w * NM + 1) * 64 + lane];
-    }
-    const int64_t t = a.t0 + r;  // lane: token column r, rows 4g + i
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const int64_t n = n0 + 4 * g + i;
         float out = sg[i];
         if (DUAL) {
             const float act = a.act == SLHIP_ACT_SILU        ? activate<SLHIP_ACT_SILU>(sg[i])
@@ -1683,8 +1189,7 @@ static void launch_mfma_lds(const MatvecArgs& a, bool dual, hipStream_t st)
     }
 }
 
-// Weight stage of the LDS-staged MFMA kernel (SLHIP_MATVEC_MFMA_SK: 256 or 512 values; 0 = operands
-// loaded straight from global memory, also used when K is not a multiple of the stage) and 16-row tiles
+// Weight stage of the LDS-staged MFMA kernel (SLHIP_MATVEC_MFMA_SK: 256 or 512 values) and 16-row tiles
 // per block (SLHIP_MATVEC_MFMA_NT: 1 or 2; one with the 512-value stage).
 static int mfma_stage() { return env_int("SLHIP_MATVEC_MFMA_SK", 256); }
 // Default: one tile (finer blocks spread the 16-row tiles more evenly over the CUs), two only for f32 x above
@@ -1699,22 +1204,12 @@ static int mfma_tiles(int64_t T, int xt)
 
 static int run_mfma(MatvecArgs a, bool dual, hipStream_t st)
 {
-    const dim3 grid(static_cast<unsigned>((a.N + 15) / 16));
     const int sk = mfma_stage(), nt = mfma_tiles(a.T, a.xt);
     for (int64_t t0 = 0; t0 < a.T; t0 += 16) {
         a.t0 = t0;
-        if (sk == 512 && a.K % 512 == 0) {
-            launch_mfma_lds<512, 1>(a, dual, st);  // two tiles would take 133 KB of LDS per block
-        } else if (sk == 256 && a.K % 256 == 0) {
-            nt == 2 ? launch_mfma_lds<256, 2>(a, dual, st) : launch_mfma_lds<256, 1>(a, dual, st);
-        } else if (a.xt == SLHIP_F32) {
-            if (dual) matvec_mfma<true, true><<<grid, 64 * kMmWaves, 0, st>>>(a);
-            else matvec_mfma<false, true><<<grid, 64 * kMmWaves, 0, st>>>(a);
-        } else {
-            if (dual) matvec_mfma<true, false><<<grid, 64 * kMmWaves, 0, st>>>(a);
-            else matvec_mfma<false, false><<<grid, 64 * kMmWaves, 0, st>>>(a);
-        }
-        const int r = check_launch("matvec_mfma");
+        if (sk == 512 && a.K % 512 == 0) launch_mfma_lds<512, 1>(a, dual, st);  // two tiles would take 133 KB of LDS per block
+        else nt == 2 ? launch_mfma_lds<256, 2>(a, dual, st) : launch_mfma_lds<256, 1>(a, dual, st);
+        const int r = check_launch("matvec_mfma_lds");
         if (r != SLHIP_OK) return r;
     }
     return SLHIP_OK;
@@ -1725,12 +1220,35 @@ static int run_mfma(MatvecArgs a, bool dual, hipStream_t st)
 // f32 x 41.6 / 44.3, bf16 x 45.1 / 40.0; at T = 3: f32 x 51.5 / 43.6.
 static int mfma_min_tokens(int xt) { return env_int("SLHIP_MATVEC_MFMA_MIN_T", xt == SLHIP_BF16 ? 2 : 3); }
 
+// Whether a bf16 launch of up to 16 tokens is faster on the LDS-staged kernel above than on matvec_kw: where
+// matvec_kw's blocks no longer go round the chip once (it then pays whole further rounds). Measured at K = 4096 (us,
+// LDS-staged / matvec_kw at 3 tokens; 16): pairs, f32 x, N = 8192 25.6 / 24.7; 32.5 / 25.6, N = 14336 44.7 / 45.7;
+// 44.6 / 50.6; pairs, bf16 x, N = 4096 15.3 / 13.3; 15.7 / 13.8, N = 6144 18.4 / 19.0; 21.0 / 19.6, N = 14336 40.0 /
+// 43.9; 43.5 / 46.6; one matrix, bf16 x, N = 14336 21.2 / 19.7; 26.5 / 20.0, N = 20480 29.3 / 34.8; 36.8 / 38.8; one
+// matrix, f32 x, N = 20480 37.8 / 36.9; 45.3 / 43.4, N = 28672 45.7 / 47.2; 59.8 / 51.7.
+static bool mfma_lds_better(const MatvecArgs& a, bool dual)
+{
+    if (a.K % 256 != 0 || a.T > 16) return false;
+    return dual ? a.N > (a.xt == SLHIP_F32 ? 8192 : 4096) : a.xt != SLHIP_F32 && a.N > 16384;
+}
+
+int run_kw(int fmt, const MatvecArgs& a, bool dual, hipStream_t st);
+
 template <int WT>
 static int run_dense(MatvecArgs a, bool dual, hipStream_t st)
 {
-    if constexpr (WT == SLHIP_BF16) {
-        const int mt = mfma_min_tokens(a.xt);
-        if (mt > 0 && a.T >= mt && a.K % 64 == 0) return run_mfma(a, dual, st);
+    if constexpr (WT != SLHIP_F32) {
+        // The matrix cores from mfma_min_tokens on; f16 weights, which take two bf16 parts, a little later with f32 x
+        // (dual at [4096, 4096] and [14336, 4096], us, VALU / matvec_kw: T = 3 18.7 / 19.5, 49.9 / 60.4; T = 5 38.0 /
+        // 19.4, 97.9 / 63.2; one matrix T = 3 12.0 / 12.8, 34.1 / 29.7); and wherever the VALU kernel cannot hold
+        // two tokens' x at once (K = 14336, N = 4096, T = 2: bf16 49.1 / 23.5, f16 50.2 / 35.6).
+        const int base = mfma_min_tokens(a.xt);
+        const int mt = WT == SLHIP_F16 && dual && a.xt == SLHIP_F32 && base > 0 ? base + 2 : base;
+        if (mt > 0 && a.K % 64 == 0 && (a.T >= mt || (a.T > 1 && token_tile(a.T, a.K) < a.T))) {
+            if (WT == SLHIP_BF16 && mfma_lds_better(a, dual)) return run_mfma(a, dual, st);
+            const int r = run_kw(WT == SLHIP_BF16 ? SLHIP_FMT_BF16 : SLHIP_FMT_F16, a, dual, st);
+            if (r != SLHIP_ERR_UNSUPPORTED) return r;
+        }
     }
     constexpr int E = Vec<WT>::N;
     const int64_t nvr = a.K / E;
@@ -1840,12 +1358,7 @@ static int quant_ch(const MatvecArgs& a, int ch, hipStream_t st)
 template <int FMT, bool DUAL>
 static int quant_tt(const MatvecArgs& a, int tt, int ch, hipStream_t st)
 {
-    switch (tt) {
-    case 1: return quant_ch<FMT, 1, DUAL>(a, ch, st);
-    case 2: return quant_ch<FMT, 2, DUAL>(a, ch, st);
-    case 4: return quant_ch<FMT, 4, DUAL>(a, ch, st);
-    default: return quant_ch<FMT, 8, DUAL>(a, ch, st);
-    }
+    return tt == 1 ? quant_ch<FMT, 1, DUAL>(a, ch, st) : quant_ch<FMT, 2, DUAL>(a, ch, st);
 }
 
 template <int FMT, bool DUAL>
@@ -1863,69 +1376,40 @@ static int launch_kq_tile(const MatvecArgs& a, hipStream_t st)
 }
 
 // Tokens from which the 32-value block formats (Q4_0, Q8_0, Q4_1, Q5_0, Q5_1) take the matrix cores
-// (SLHIP_MATVEC_MQ_MIN_T; 0 disables). Measured with matvec_mq2 at [14336, 4096] (dual, f32 x, us, VALU /
-// matrix cores): Q4_0 T = 2 28.1 / 44.1, T = 3 56.8 / 45.0; Q8_0 T = 2 32.5 / 46.2, T = 3 58.0 / 48.1.
+// (SLHIP_MATVEC_MQ_MIN_T; 0 disables). Measured at [14336, 4096] (dual, f32 x, us, VALU / matrix cores): Q4_0 T = 2
+// 28.1 / 44.1, T = 3 56.8 (in one pass of four) / 29.6; Q8_0 T = 2 32.5 / 46.2, T = 3 58.0 / 31.0.
 static int mq_min_tokens() { return env_int("SLHIP_MATVEC_MQ_MIN_T", 3); }
-// The same for the K-quants (SLHIP_MATVEC_KQ_MIN_T). With matvec_mq2, measured dual at [14336, 4096], f32 x
-// (us, VALU / matrix cores): Q4_K T = 2 30.6 / 46.5, T = 3 60.6 / 49.0; Q6_K T = 3 94.2 / 62.5; Q3_K T = 3
-// 78.0 / 61.2 (the VALU kernel's passes hold 2 and then 4 tokens): from three tokens.
+// The same for the K-quants (SLHIP_MATVEC_KQ_MIN_T). Measured dual at [14336, 4096], f32 x (us, VALU / matrix cores):
+// Q4_K T = 2 26.8 / 31.1, T = 3 60.6 / 31.5; Q6_K T = 2 35.3 / 54.4, T = 3 94.2 / 54.6; Q3_K T = 3 78.0 / 46.8.
 static int kq_min_tokens() { return env_int("SLHIP_MATVEC_KQ_MIN_T", 3); }
 
-// The several-token kernel with the stage moved straight to LDS and each lane scaling its own row
-// (matvec_mq.hpp, matvec_mq_*.hip); SLHIP_MATVEC_MQ2=0 keeps matvec_mfma_q below, which also takes the
-// launches mq2 does not fit.
-int run_mq2_part0(int fmt, const MatvecArgs& a, bool dual, hipStream_t st);
-int run_mq2_part1(int fmt, const MatvecArgs& a, bool dual, hipStream_t st);
-int run_mq2_part2(int fmt, const MatvecArgs& a, bool dual, hipStream_t st);
-
-static int run_mq2_any(int fmt, const MatvecArgs& a, bool dual, hipStream_t st)
+// matvec_mq2 (matvec_mq.hpp): the 32-value block formats at up to 16 tokens where matvec_kw's blocks go round the chip
+// more than once: pairs of more than 4096 rows, one matrix of more than 16384 (Q8_0: 8192). Measured at K = 4096, f32 x
+// (us, mq2 / matvec_kw at 3 tokens; 16): pairs Q4_0 N = 4096 19.3 / 13.6; 20.1 / 15.1, N = 6144 18.8 / 19.7; 20.2 /
+// 20.3, N = 14336 29.6 / 38.2; 33.0 / 39.5; Q8_0 N = 4096 18.7 / 15.0; 20.9 / 17.0, N = 6144 19.9 / 22.3; 21.1 / 23.1,
+// N = 14336 31.0 / 45.0; 34.1 / 47.4; one matrix Q4_0 N = 14336 20.3 / 20.2; 23.6 / 20.8, N = 20480 28.4 / 35.0; 32.4 /
+// 38.1; Q8_0 N = 8192 13.4 / 14.8; 16.0 / 15.9, N = 14336 20.1 / 23.9; 24.9 / 25.1.
+int run_mq2_any(int fmt, const MatvecArgs& a, bool dual, hipStream_t st);
+static bool mq2_better(int fmt, const MatvecArgs& a, bool dual)
 {
-    switch (fmt) {
-    case SLHIP_FMT_Q4_0:
-    case SLHIP_FMT_Q8_0:
-    case SLHIP_FMT_Q4_1:
-    case SLHIP_FMT_Q5_0:
-    case SLHIP_FMT_Q5_1: return run_mq2_part0(fmt, a, dual, st);
-    case SLHIP_FMT_Q4_K:
-    case SLHIP_FMT_Q5_K: return run_mq2_part1(fmt, a, dual, st);
-    default: return run_mq2_part2(fmt, a, dual, st);
-    }
-}
-
-template <int FMT>
-static int run_mfma_q(MatvecArgs a, bool dual, hipStream_t st)
-{
-    if (env_int("SLHIP_MATVEC_MQ2", 1)) {
-        const int r = run_mq2_any(FMT, a, dual, st);
-        if (r != SLHIP_ERR_UNSUPPORTED) return r;
-    }
-    const dim3 grid(static_cast<unsigned>((a.N + 15) / 16));
-    for (int64_t t0 = 0; t0 < a.T; t0 += 16) {
-        a.t0 = t0;
-        if (a.xt == SLHIP_F32) {
-            if (dual) matvec_mfma_q<FMT, true, true><<<grid, 64 * kMqWaves, 0, st>>>(a);
-            else matvec_mfma_q<FMT, false, true><<<grid, 64 * kMqWaves, 0, st>>>(a);
-        } else {
-            if (dual) matvec_mfma_q<FMT, true, false><<<grid, 64 * kMqWaves, 0, st>>>(a);
-            else matvec_mfma_q<FMT, false, false><<<grid, 64 * kMqWaves, 0, st>>>(a);
-        }
-        const int r = check_launch("matvec_mfma_q");
-        if (r != SLHIP_OK) return r;
-    }
-    return SLHIP_OK;
+    return a.T <= 16 && a.N > (dual ? 4096 : fmt == SLHIP_FMT_Q8_0 ? 8192 : 16384);
 }
 
 template <int FMT>
 static int run_quant(MatvecArgs a, bool dual, hipStream_t st)
 {
-    if constexpr (FMT == SLHIP_FMT_Q4_0 || FMT == SLHIP_FMT_Q8_0 || FMT == SLHIP_FMT_Q4_1 || FMT == SLHIP_FMT_Q5_0 ||
-                  FMT == SLHIP_FMT_Q5_1 || FMT == SLHIP_FMT_Q4_K || FMT == SLHIP_FMT_Q5_K || FMT == SLHIP_FMT_Q6_K ||
-                  FMT == SLHIP_FMT_Q2_K || FMT == SLHIP_FMT_Q3_K) {
-        // several tokens: the matrix-core kernel, when K splits into whole stages (and the rows into its loads)
-        const int mt = Fmt<FMT>::K ? kq_min_tokens() : mq_min_tokens();
-        const uintptr_t al = reinterpret_cast<uintptr_t>(a.wg) | reinterpret_cast<uintptr_t>(a.wu);
-        if (mt > 0 && a.T >= mt && a.K % (MqGeom<FMT>::SKB * 32) == 0 && al % MqGeom<FMT>::UB == 0)
-            return run_mfma_q<FMT>(a, dual, st);
+    // Several tokens: the matrix cores; at two tokens only where the VALU kernel cannot hold both tokens' x in LDS
+    // (K = 14336, N = 4096, us, VALU / matvec_kw: Q4_K 38.6 / 22.0, Q6_K 76 / 30, Q8_0 38.9 / 25.4).
+    const int mt = Fmt<FMT>::K ? kq_min_tokens() : mq_min_tokens();
+    if (mt > 0 && (a.T >= mt || (a.T > 1 && quant_lds(2, a.K, a.wrow, dual) > kMaxLds))) {
+        if constexpr (!Fmt<FMT>::K) {
+            if (mq2_better(FMT, a, dual)) {
+                const int r = run_mq2_any(FMT, a, dual, st);
+                if (r != SLHIP_ERR_UNSUPPORTED) return r;
+            }
+        }
+        const int r = run_kw(FMT, a, dual, st);
+        if (r != SLHIP_ERR_UNSUPPORTED) return r;
     }
     if constexpr (FMT == SLHIP_FMT_Q4_K || FMT == SLHIP_FMT_Q6_K) {
         // one token: the matrix-core kernel, when K splits into whole segments and its LDS fits
@@ -1933,8 +1417,7 @@ static int run_quant(MatvecArgs a, bool dual, hipStream_t st)
             env_int("SLHIP_KQ_MFMA", 1))
             return dual ? launch_kq_tile<FMT, true>(a, st) : launch_kq_tile<FMT, false>(a, st);
     }
-    int tt = Fmt<FMT>::K && dual ? 4 : 8;  // the K-quant sub-block decode at 8 tokens of a pair spills
-    while (tt > 1 && (tt / 2 >= a.T || quant_lds(tt, a.K, a.wrow, dual) > kMaxLds)) tt /= 2;
+    const int tt = a.T > 1 && quant_lds(2, a.K, a.wrow, dual) <= kMaxLds ? 2 : 1;
     if (quant_lds(tt, a.K, a.wrow, dual) > kMaxLds)
         return fail(SLHIP_ERR_UNSUPPORTED, "matvec: K = %lld does not fit in LDS for this format", static_cast<long long>(a.K));
     const int64_t per_lane = ((dual ? 2 : 1) * (a.wrow / 16) + 63) / 64;

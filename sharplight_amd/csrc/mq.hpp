@@ -1,6 +1,6 @@
 #pragma once
-// Pieces shared by the matvec kernels (matvec.hip) and the several-token block-format kernel on the bf16
-// matrix cores (matvec_mq.hpp): the launch arguments, x split into bf16 parts, the per-format stage geometry
+// Pieces shared by the matvec kernels (matvec.hip) and the several-token kernels on the bf16 matrix cores
+// (matvec_kw.hpp, matmul_tile.hpp, matvec_mq.hpp): the launch arguments, x split into bf16 parts, the per-format stage geometry
 // and the block formats' codes as exact bf16 operands.
 #include "act.hpp"
 #include "common.hpp"
@@ -68,18 +68,12 @@ __device__ __forceinline__ void split3(const float* x, uint4& h, uint4& m, uint4
 }
 
 template <int FMT> struct MqGeom;
-constexpr int kMqWaves = 8;
 // SKB: 32-value blocks per stage, RB: bytes of one row per stage, UB: bytes per staging load
 template <> struct MqGeom<SLHIP_FMT_Q4_0> { static constexpr int SKB = 32, RB = 32 * 18, UB = 16; };
 template <> struct MqGeom<SLHIP_FMT_Q8_0> { static constexpr int SKB = 16, RB = 16 * 34, UB = 16; };
 template <> struct MqGeom<SLHIP_FMT_Q4_1> { static constexpr int SKB = 32, RB = 32 * 20, UB = 16; };
 template <> struct MqGeom<SLHIP_FMT_Q5_0> { static constexpr int SKB = 32, RB = 32 * 22, UB = 16; };
 template <> struct MqGeom<SLHIP_FMT_Q5_1> { static constexpr int SKB = 32, RB = 32 * 24, UB = 16; };
-template <> struct MqGeom<SLHIP_FMT_Q4_K> { static constexpr int SKB = 32, RB = 4 * 144, UB = 16; };  // 4 super-blocks
-template <> struct MqGeom<SLHIP_FMT_Q5_K> { static constexpr int SKB = 32, RB = 4 * 176, UB = 16; };
-template <> struct MqGeom<SLHIP_FMT_Q6_K> { static constexpr int SKB = 16, RB = 2 * 210, UB = 4; };   // 420 bytes
-template <> struct MqGeom<SLHIP_FMT_Q2_K> { static constexpr int SKB = 32, RB = 4 * 84, UB = 16; };   // 336 bytes
-template <> struct MqGeom<SLHIP_FMT_Q3_K> { static constexpr int SKB = 32, RB = 4 * 110, UB = 8; };   // 440 bytes
 
 // Eight codes of lane group g (values 8g .. 8g + 7 of the block) as four bf16 pairs, the format's offset
 // applied (Q4_0 q - 8, Q5_0 q - 16: exact); row: the row's stage bytes (4-byte aligned), off: the block's
@@ -136,22 +130,16 @@ __device__ __forceinline__ uint4 mq_codes(const uint8_t* row, int off, int g)
     return make_uint4(pack_bf16x2(f[0], f[1]), pack_bf16x2(f[2], f[3]), pack_bf16x2(f[4], f[5]), pack_bf16x2(f[6], f[7]));
 }
 
-// Eight Q4_K codes of lane group g (values 8g .. 8g + 7 of sub-block j: the low (j even) or high nibbles of
-// bytes 32 (j / 2) + 8g .. of the super-block's 128 code bytes, Quant.cs:518-545) as four bf16 pairs; sbo: the
-// super-block's first byte in the staged row (a multiple of 16), so the eight bytes are one aligned 8-byte read.
-// Q5_K (FIVE): the codes after a 32-byte qh at byte 16, and value l of sub-block j adds 16 when bit j of qh[l]
-// is set (ggml's Q5_K layout, the same scale packing as Q4_K).
-template <bool FIVE = false>
-__device__ __forceinline__ uint4 q4k_codes(const uint8_t* row, int sbo, int j, int g)
+// Eight Q5_K codes of lane group g (values 8g .. 8g + 7 of sub-block j of the super-block at `row`, 16-byte aligned) as
+// four bf16 pairs: the low (j even) or high nibbles of bytes 32 (j / 2) + 8g .. of the 128 code bytes at 48, plus 16
+// when bit j of byte l of the 32-byte qh at 16 is set (ggml's Q5_K layout).
+__device__ __forceinline__ uint4 q5k_codes(const uint8_t* row, int j, int g)
 {
-    const uint2 w = *reinterpret_cast<const uint2*>(row + sbo + (FIVE ? 48 : 16) + 32 * (j >> 1) + 8 * g);
+    const uint2 w = *reinterpret_cast<const uint2*>(row + 48 + 32 * (j >> 1) + 8 * g);
+    const uint2 h = *reinterpret_cast<const uint2*>(row + 16 + 8 * g);
     const uint32_t sh = 4 * static_cast<uint32_t>(j & 1);
-    uint32_t lo = (w.x >> sh) & 0x0F0F0F0Fu, hi = (w.y >> sh) & 0x0F0F0F0Fu;
-    if constexpr (FIVE) {
-        const uint2 h = *reinterpret_cast<const uint2*>(row + sbo + 16 + 8 * g);
-        lo |= ((h.x >> j) & 0x01010101u) << 4;
-        hi |= ((h.y >> j) & 0x01010101u) << 4;
-    }
+    const uint32_t lo = ((w.x >> sh) & 0x0F0F0F0Fu) | (((h.x >> j) & 0x01010101u) << 4);
+    const uint32_t hi = ((w.y >> sh) & 0x0F0F0F0Fu) | (((h.y >> j) & 0x01010101u) << 4);
     float f[8];
 #pragma unroll
     for (int e = 0; e < 4; e++) {
@@ -170,53 +158,30 @@ __device__ __forceinline__ uint2 lds_bytes8(const uint8_t* row, int q)
     return make_uint2(__builtin_amdgcn_alignbit(w1, w0, sh), __builtin_amdgcn_alignbit(w2, w1, sh));
 }
 
-// Eight Q2_K / Q3_K codes of lane group g for the 32-value block u = 4n + j of a super-block, as four bf16
-// pairs (Quant.KQuants.cs:36-107, ggml's layouts): value 128n + 32j + 8g + e has the 2-bit field 2j of byte
-// 32n + 8g + e of qs (Q2_K: qs at 16; Q3_K: qs at 32, plus 4 when bit 4n + j of hmask byte 8g + e is set,
-// minus 4). Lane groups 0-1 hold the block's first 16-value scale group, 2-3 the second.
-template <bool Q3>
-__device__ __forceinline__ uint4 q23k_codes(const uint8_t* row, int sbo, int u, int g)
-{
-    const int n = u >> 2, j = u & 3;
-    const uint2 l = lds_bytes8(row, sbo + (Q3 ? 32 : 16) + 32 * n + 8 * g);
-    const uint32_t sh = 2 * static_cast<uint32_t>(j);
-    uint32_t q0 = (l.x >> sh) & 0x03030303u, q1 = (l.y >> sh) & 0x03030303u;
-    if constexpr (Q3) {
-        const uint2 h = lds_bytes8(row, sbo + 8 * g);
-        const uint32_t hs = static_cast<uint32_t>(4 * n + j);
-        q0 |= ((h.x >> hs) & 0x01010101u) << 2;
-        q1 |= ((h.y >> hs) & 0x01010101u) << 2;
-    }
-    constexpr float OFF = Q3 ? -4.0f : 0.0f;
-    float f[8];
-#pragma unroll
-    for (int e = 0; e < 4; e++) {
-        f[e] = static_cast<float>((q0 >> (8 * e)) & 0xFFu) + OFF;
-        f[4 + e] = static_cast<float>((q1 >> (8 * e)) & 0xFFu) + OFF;
-    }
-    return make_uint4(pack_bf16x2(f[0], f[1]), pack_bf16x2(f[2], f[3]), pack_bf16x2(f[4], f[5]), pack_bf16x2(f[6], f[7]));
-}
-
-// The same eight Q2_K / Q3_K codes multiplied by the integer scale of their 16-value group (lane groups 0-1: the
+// Eight Q2_K / Q3_K codes of lane group g for the 32-value block u = 4n + j of a super-block (Quant.KQuants.cs:36-107,
+// ggml's layouts): value 128n + 32j + 8g + e has the 2-bit field 2j of byte 32n + 8g + e of qs (Q2_K: qs at 16; Q3_K: qs
+// at 32, plus 4 when bit 4n + j of hmask byte 8g + e is set, minus 4), multiplied by the integer scale of their
+// 16-value group (lane groups 0-1: the
 // block's first group, 2-3 its second), with the super-block's d: d * (code * scale) is the weight, and
 // code * scale is an exact bf16 integer (Q3_K |(q - 4) * (s - 32)| <= 128, Q2_K q * s <= 45), so that both
 // groups of a block take one MFMA chain (Quant.KQuants.cs:36-107: Q3_K scales are 6-bit fields, 4 low bits at
 // byte 96 + (i % 8), 2 high bits at byte 104 + i % 4, minus 32; Q2_K's are the low nibbles of bytes 0..15).
+// ts: how much further in the image the fields past the codes sit (Q3_K from byte 96, Q2_K from byte 80).
 template <bool Q3>
-__device__ __forceinline__ uint4 q23k_codes_scaled(const uint8_t* row, int sbo, int u, int g, float& d)
+__device__ __forceinline__ uint4 q23k_codes_scaled(const uint8_t* row, int sbo, int u, int g, float& d, int ts = 0)
 {
     auto u16 = [&](int o) { return static_cast<uint32_t>(*reinterpret_cast<const uint16_t*>(row + o)); };
     float sc;
     if constexpr (Q3) {
-        d = static_cast<float>(*reinterpret_cast<const _Float16*>(row + sbo + 108));
+        d = static_cast<float>(*reinterpret_cast<const _Float16*>(row + sbo + ts + 108));
         const int s0 = 2 * u, w = s0 >> 2, b0 = s0 & 3;
-        const uint32_t a = u16(sbo + 96 + 4 * (w & 1) + b0);
-        const uint32_t h = u16(sbo + 104 + b0);
+        const uint32_t a = u16(sbo + ts + 96 + 4 * (w & 1) + b0);
+        const uint32_t h = u16(sbo + ts + 104 + b0);
         const uint32_t lo = w < 2 ? (a & 0x0F0Fu) : ((a >> 4) & 0x0F0Fu);
         const uint32_t s2 = lo | (((h >> (2 * w)) & 0x0303u) << 4);
         sc = static_cast<float>(static_cast<int>(g < 2 ? (s2 & 0xFFu) : (s2 >> 8)) - 32);
     } else {
-        d = static_cast<float>(*reinterpret_cast<const _Float16*>(row + sbo + 80));
+        d = static_cast<float>(*reinterpret_cast<const _Float16*>(row + sbo + ts + 80));
         const uint32_t v = u16(sbo + 2 * u);
         sc = static_cast<float>(g < 2 ? (v & 0xFu) : ((v >> 8) & 0xFu));
     }
