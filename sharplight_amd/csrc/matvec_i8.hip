@@ -96,7 +96,11 @@ __global__ __launch_bounds__(256) void quantize_q8(const void* x, int64_t xs, in
             make_float4(d, __fmul_rn(d, static_cast<float>(s)), __fmul_rn(d, static_cast<float>(s_hi)), 0.0f);
 }
 
-bool matvec_q8_supported(int fmt) { return i8_geom(fmt).bs != 0; }
+// instantiated in matvec_kw8_*.hip
+int launch_kw8_part0(int fmt, const I8Args& a, bool dual, int tn, hipStream_t st);
+int launch_kw8_part1(int fmt, const I8Args& a, bool dual, int tn, hipStream_t st);
+int launch_kw8_part2(int fmt, const I8Args& a, bool dual, int tn, hipStream_t st);
+int launch_kw8_part3(int fmt, const I8Args& a, bool dual, int tn, hipStream_t st);
 
 bool matvec_q8_fits(int fmt, int64_t K, bool dual)
 {
@@ -104,6 +108,53 @@ bool matvec_q8_fits(int fmt, int64_t K, bool dual)
     if (g.bs == 0 || K <= 0 || K % g.bs != 0 || (K / g.bs * g.bb) % 2 != 0) return false;
     return i8_lds(1, K, K / g.bs * g.bb, dual) <= kI8MaxLds;
 }
+
+// Whether matvec_kw8 takes the call: 0, or the row tiles of its blocks. The other kernels keep a group's rows resident
+// and loop over few tokens, so they win at few tokens and wherever the rows alone fill the chip several times over; they
+// pay K long (x leaves LDS to few tokens), few rows (idle CUs) and every 16 tokens again. g: 16-row groups, both matrices
+// counted. Q4_K, K = 4096, us here / there: N = 4096 8.4 / 13 (T = 4), 8.4 / 16 (T = 16), 10.4 / 28 (T = 31); N = 14336
+// 14.7 / 15.2, 15.1 / 20, 21.8 / 37; K = 14336, N = 4096 15 / 33, 16 / 42, 21 / 81; T = 2: 8.5 / 8.6. Past the lines
+// below: dual Q4_K, N = 14336 (g = 1792) 23.6 / 21.9 (T = 4), 23.6 / 22.8 (T = 8); Q6_K, N = 14336 21.8 / 16.7 (T = 3);
+// Q8_0 dual, K = 2048, N = 8192 (g = 1024) 16.3 / 13.7 (T = 16); Q5_1, N = 128256 251 / 223 (T = 31).
+static int kw8_tiles(int fmt, const I8Args& a, bool dual)
+{
+    const int env = i8_mfma_env();
+    if (a.K % 256 != 0 || env == 0 || a.T < env || !matvec_q8_fits(fmt, a.K, dual)) return 0;
+    const int64_t rows = (a.N + 15) / 16, g = dual ? 2 * rows : rows;
+    const bool small = kw8_two_tiles(fmt);
+    bool take;
+    if (a.T > 16)
+        take = g <= 2048 || (fmt != SLHIP_FMT_Q5_0 && fmt != SLHIP_FMT_Q5_1);
+    else if (small)
+        take = g <= 1024 ? a.T >= 3 : !dual && a.T > 8;
+    else if (a.wrow % 16 != 0)  // (the other kernels' matrix-core forms want 16-byte rows)
+        take = a.T >= 5;
+    else
+        take = g <= (dual ? 512 : 1024) && a.T >= (a.K >= 8192 ? 4 : 5);
+    if (!take) return 0;
+    // two tiles a block where one each would be more than two blocks a CU: N = 14336, T = 16 15.1 / 17.7; N = 4096 9.7 / 8.4
+    return small && !dual && rows * ((a.T + 15) / 16) > 512 ? 2 : 1;
+}
+
+static int run_kw8(int fmt, const I8Args& a, bool dual, hipStream_t st)
+{
+    const int tn = kw8_tiles(fmt, a, dual);
+    if (tn == 0) return SLHIP_ERR_UNSUPPORTED;
+    switch (fmt) {
+    case SLHIP_FMT_Q4_K:
+    case SLHIP_FMT_Q5_K: return launch_kw8_part0(fmt, a, dual, tn, st);
+    case SLHIP_FMT_Q6_K:
+    case SLHIP_FMT_Q8_0: return launch_kw8_part1(fmt, a, dual, tn, st);
+    case SLHIP_FMT_Q4_0:
+    case SLHIP_FMT_Q4_1: return launch_kw8_part2(fmt, a, dual, tn, st);
+    case SLHIP_FMT_Q5_0:
+    case SLHIP_FMT_Q5_1:
+    case SLHIP_FMT_IQ4_NL: return launch_kw8_part3(fmt, a, dual, tn, st);
+    default: return SLHIP_ERR_UNSUPPORTED;
+    }
+}
+
+bool matvec_q8_supported(int fmt) { return i8_geom(fmt).bs != 0; }
 
 int quantize_q8_common(int dtype_x, const void* x, int64_t x_stride, int64_t T, int64_t K, void* xq, hipStream_t st)
 {
@@ -149,6 +200,8 @@ int matvec_q8_common(int fmt, int dtype_y, const void* xq, int64_t T, int64_t K,
     if (N > 0x7FFFFFFF || T > 0x7FFFFFFF) return fail(SLHIP_ERR_UNSUPPORTED, "%s: shape too large", name);
     I8Args a{static_cast<const uint8_t*>(xq), static_cast<const char*>(wg), static_cast<const char*>(wu),
              K / g.bs * g.bb, y, y_stride, T, K, N, 0, dtype_y, act, dual ? nullptr : bias};
+    const int r8 = run_kw8(fmt, a, dual, st);
+    if (r8 != SLHIP_ERR_UNSUPPORTED) return r8;
     switch (fmt) {
     case SLHIP_FMT_Q8_0:
     case SLHIP_FMT_Q4_0:

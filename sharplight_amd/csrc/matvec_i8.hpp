@@ -1044,14 +1044,20 @@ static int i8_tt(const I8Args& a, int tt, hipStream_t st)
 // 27.3 -> 31.0 / 28.1 / 26.4; Q5_0 / Q5_1 / IQ4_XS level or behind at T4 and Q6_K 37.4 -> 53.2, so those from
 // 5 (where the VALU kernel takes an 8-token pass and falls 1.6-1.9x behind). SLHIP_MATVEC_I8_MFMA_MIN_T
 // overrides it for every format (0 disables).
-template <int FMT>
-inline int i8_mfma_min_tokens()
+inline int i8_mfma_env()  // the variable's value, -1 if unset
 {
     static int v = -2;
     if (v == -2) {
         const char* e = getenv("SLHIP_MATVEC_I8_MFMA_MIN_T");
         v = e ? atoi(e) : -1;
     }
+    return v;
+}
+
+template <int FMT>
+inline int i8_mfma_min_tokens()
+{
+    const int v = i8_mfma_env();
     if (v != -1) return v;
     switch (FMT) {
     case SLHIP_FMT_Q8_0:
@@ -1100,6 +1106,10 @@ int run_i8(I8Args a, bool dual, hipStream_t st)
     }
     return SLHIP_OK;
 }
+
+// matvec_kw8: the formats whose two-tile blocks leave LDS for a second block on the CU (the others' do not, and lose to
+// one tile).
+constexpr bool kw8_two_tiles(int fmt) { return fmt == SLHIP_FMT_Q4_K || fmt == SLHIP_FMT_Q4_0 || fmt == SLHIP_FMT_IQ4_NL; }
 
 // instantiated in matvec_i8_*.hip, one group of formats per unit
 int run_i8_part0(int fmt, const I8Args& a, bool dual, hipStream_t st);

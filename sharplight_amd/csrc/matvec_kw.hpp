@@ -267,8 +267,8 @@ __device__ __forceinline__ float x_parts(const float (&v)[8], uint4* P)
 }
 
 // y[t, n] from the finished sums of one output (gate and up for the dual form).
-template <bool DUAL>
-__device__ __forceinline__ void store_sum(const MatvecArgs& a, int64_t t, int64_t n, float sg, float su)
+template <bool DUAL, class Args>
+__device__ __forceinline__ void store_sum(const Args& a, int64_t t, int64_t n, float sg, float su)
 {
     float out = sg;
     if (DUAL) {
@@ -283,6 +283,42 @@ __device__ __forceinline__ void store_sum(const MatvecArgs& a, int64_t t, int64_
             static_cast<float*>(a.y)[t * a.ys + n] = out;
         else
             static_cast<uint16_t*>(a.y)[t * a.ys + n] = static_cast<uint16_t>(f32_to_bf16_bits(out));
+    }
+}
+
+// The waves' partial sums of a block's tiles meet in the (now idle) stage memory, up to 4 output tiles per round:
+// [wave][tile][matrix][lane]; wave q finishes tile q of the round.
+template <bool DUAL, int MT, int TN, int G, class Args>
+__device__ __forceinline__ void reduce_store(const Args& a, const f32x4_t (&acc)[G][MT], uint8_t* lds, int wave, int lane,
+                                             int64_t n0, int64_t t0)
+{
+    constexpr int NM = DUAL ? 2 : 1, UN = TN * MT, UR = UN < 4 ? UN : 4;
+    const int r = lane & 15, g = lane >> 4;
+    f32x4_t* red = reinterpret_cast<f32x4_t*>(lds);
+#pragma unroll
+    for (int q0 = 0; q0 < UN; q0 += UR) {
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < UR; q++)
+#pragma unroll
+            for (int m = 0; m < NM; m++)
+                red[((wave * UR + q) * NM + m) * 64 + lane] = acc[m * TN + (q0 + q) / MT][(q0 + q) % MT];
+        __syncthreads();
+        if (wave < UR) {
+            f32x4_t sg = red[(wave * NM) * 64 + lane], su = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+            if (DUAL) su = red[(wave * NM + NM - 1) * 64 + lane];
+#pragma unroll
+            for (int v = 1; v < kKwWaves; v++) {
+                sg += red[((v * UR + wave) * NM) * 64 + lane];
+                if (DUAL) su += red[((v * UR + wave) * NM + NM - 1) * 64 + lane];
+            }
+            const int64_t n = n0 + 16 * ((q0 + wave) / MT) + r;
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int64_t t = t0 + 16 * ((q0 + wave) % MT) + 4 * g + i;
+                store_sum<DUAL>(a, t, n, sg[i], su[i]);
+            }
+        }
     }
 }
 
@@ -383,11 +419,13 @@ __global__ __launch_bounds__(64 * kKwWaves) __attribute__((amdgpu_waves_per_eu(2
         for (int u = 0; u < PD; u++) load_x((s0 * SKB + u) * 32, u);
 
         for (int s = s0; s < s1; s++) {
+            wave_lds_sync();  // the previous stage's reads, by every lane, come first
 #pragma unroll
             for (int m = 0; m < NM; m++)
 #pragma unroll
                 for (int i = 0; i < NL; i++)
                     *reinterpret_cast<uint4*>(img + m * (16 * TN * Geo::PITCH) + dst[i]) = w[m][i];
+            wave_lds_sync();
             const int sn = s + 1 < s1 ? s + 1 : s;  // (the last stage's loads again: a fixed number of loads per stage)
             __builtin_amdgcn_sched_barrier(0);
             load_w(sn);
@@ -464,34 +502,7 @@ __global__ __launch_bounds__(64 * kKwWaves) __attribute__((amdgpu_waves_per_eu(2
         }
     }
 
-    // The waves' partial sums meet in the (now idle) stage memory, UR output tiles per round: [wave][tile][matrix][lane];
-    // wave q finishes tile q of the round.
-    f32x4_t* red = reinterpret_cast<f32x4_t*>(lds);
-#pragma unroll
-    for (int q0 = 0; q0 < UN; q0 += UR) {
-        __syncthreads();
-#pragma unroll
-        for (int q = 0; q < UR; q++)
-#pragma unroll
-            for (int m = 0; m < NM; m++)
-                red[((wave * UR + q) * NM + m) * 64 + lane] = acc[m * TN + (q0 + q) / MT][(q0 + q) % MT];
-        __syncthreads();
-        if (wave < UR) {
-            f32x4_t sg = red[(wave * NM) * 64 + lane], su = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-            if (DUAL) su = red[(wave * NM + NM - 1) * 64 + lane];
-#pragma unroll
-            for (int v = 1; v < kKwWaves; v++) {
-                sg += red[((v * UR + wave) * NM) * 64 + lane];
-                if (DUAL) su += red[((v * UR + wave) * NM + NM - 1) * 64 + lane];
-            }
-            const int64_t n = n0 + 16 * ((q0 + wave) / MT) + r;
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int64_t t = t0 + 16 * ((q0 + wave) % MT) + 4 * g + i;
-                store_sum<DUAL>(a, t, n, sg[i], su[i]);
-            }
-        }
-    }
+    reduce_store<DUAL, MT, TN>(a, acc, lds, wave, lane, n0, t0);
 }
 
 template <int FMT, bool DUAL, bool XF32, int MT, int TN>

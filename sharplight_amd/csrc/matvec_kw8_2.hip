@@ -1,0 +1,15 @@
+// Instantiations of matvec_kw8 for Q4_0 and Q4_1 (units of their own so that the formats compile in parallel).
+#include "matvec_kw8.hpp"
+
+namespace slhip {
+
+int launch_kw8_part2(int fmt, const I8Args& a, bool dual, int tn, hipStream_t st)
+{
+    switch (fmt) {
+    case SLHIP_FMT_Q4_0: return launch_kw8_fmt<SLHIP_FMT_Q4_0>(a, dual, tn, st);
+    case SLHIP_FMT_Q4_1: return launch_kw8_fmt<SLHIP_FMT_Q4_1>(a, dual, tn, st);
+    default: return SLHIP_ERR_UNSUPPORTED;
+    }
+}
+
+}  // namespace slhip
