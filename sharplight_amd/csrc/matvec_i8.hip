@@ -113,9 +113,9 @@ bool matvec_q8_fits(int fmt, int64_t K, bool dual)
 // and loop over few tokens, so they win at few tokens and wherever the rows alone fill the chip several times over; they
 // pay K long (x leaves LDS to few tokens), few rows (idle CUs) and every 16 tokens again. g: 16-row groups, both matrices
 // counted. Q4_K, K = 4096, us here / there: N = 4096 8.4 / 13 (T = 4), 8.4 / 16 (T = 16), 10.4 / 28 (T = 31); N = 14336
-// 14.7 / 15.2, 15.1 / 20, 21.8 / 37; K = 14336, N = 4096 15 / 33, 16 / 42, 21 / 81; T = 2: 8.5 / 8.6. Past the lines
-// below: dual Q4_K, N = 14336 (g = 1792) 23.6 / 21.9 (T = 4), 23.6 / 22.8 (T = 8); Q6_K, N = 14336 21.8 / 16.7 (T = 3);
-// Q8_0 dual, K = 2048, N = 8192 (g = 1024) 16.3 / 13.7 (T = 16); Q5_1, N = 128256 251 / 223 (T = 31).
+// 14.5 / 15.2, 14.9 / 20, 21.4 / 37; K = 14336, N = 4096 15 / 33, 16 / 42, 21 / 81; T = 2: 8.5 / 8.6; dual, N = 14336
+// (g = 1792) 23.6 / 25.8 (T = 16). Past the lines below: the same 23 / 21.9 (T = 4), 23 / 22.8 (T = 8); Q6_K, N = 14336
+// 21.8 / 16.7 (T = 3); Q8_0 dual, K = 2048, N = 8192 (g = 1024) 16.3 / 13.7 (T = 16); Q5_1, N = 128256 251 / 223 (T = 31).
 static int kw8_tiles(int fmt, const I8Args& a, bool dual)
 {
     const int env = i8_mfma_env();
@@ -126,7 +126,7 @@ static int kw8_tiles(int fmt, const I8Args& a, bool dual)
     if (a.T > 16)
         take = g <= 2048 || (fmt != SLHIP_FMT_Q5_0 && fmt != SLHIP_FMT_Q5_1);
     else if (small)
-        take = g <= 1024 ? a.T >= 3 : !dual && a.T > 8;
+        take = a.T >= (g <= 1024 ? 3 : 9);
     else if (a.wrow % 16 != 0)  // (the other kernels' matrix-core forms want 16-byte rows)
         take = a.T >= 5;
     else

@@ -426,9 +426,9 @@ __global__ __launch_bounds__(64 * kKwWaves) __attribute__((amdgpu_waves_per_eu(2
                 for (int i = 0; i < NL; i++)
                     *reinterpret_cast<uint4*>(img + m * (16 * TN * Geo::PITCH) + dst[i]) = w[m][i];
             wave_lds_sync();
-            const int sn = s + 1 < s1 ? s + 1 : s;  // (the last stage's loads again: a fixed number of loads per stage)
+            const int sn = s + 1 < s1 ? s + 1 : s;  // (x: the last stage's blocks again)
             __builtin_amdgcn_sched_barrier(0);
-            load_w(sn);
+            if (s + 1 < s1) load_w(sn);  // (two stages a wave at K = 4096: not the last one again; 14336 rows -1 to -6 %)
             __builtin_amdgcn_sched_barrier(0);
             KwScales<FMT> ks[G];
             float xs0[MT], xs1[MT];
