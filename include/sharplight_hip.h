@@ -601,7 +601,8 @@ SLHIP_API int slhip_node_supports(const char* segment_ir, int node_index, int* s
 /* IComputeDevice.Compile (IComputeDevice.cs:33-38): allocates every value for max_tokens tokens
  * (CompileOptions.MaxTokens, 0 .. 2^20). SLHIP_ERR_UNSUPPORTED for a node or pattern this provider cannot run. */
 SLHIP_API int slhip_segment_compile(const char* segment_ir, int64_t max_tokens, slhip_segment* segment);
-/* ICompiledSegment.SetInput (ICompiledSegment.cs:9-10): dense host bytes of an input or weight value. */
+/* ICompiledSegment.SetInput (ICompiledSegment.cs:9-10): dense host bytes of an input or weight value, taken before the
+ * call returns. Raises the error of an earlier run that nothing has waited for. */
 SLHIP_API int slhip_segment_set_input(slhip_segment segment, int value, const void* data, size_t bytes);
 /* ICompiledSegment.Execute: runs the launches for `tokens` tokens; asynchronous until an output is read.
  * A token count above the compiled bound fails like CpuCompiledSegment.Execute

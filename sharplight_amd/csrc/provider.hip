@@ -39,6 +39,7 @@
 #include <tuple>
 #include <map>
 #include <memory>
+#include <mutex>
 #include <set>
 #include <sstream>
 #include <stdexcept>
@@ -696,6 +697,7 @@ public:
 
     ~Segment()
     {
+        if (stage_.base && stream_) slhip_stream_sync(stream_);
         for (auto& kv : mem_) slhip_free(kv.second);
         for (void* p : scratch_) slhip_free(p);
         if (stream_) slhip_stream_destroy(stream_);
@@ -709,8 +711,22 @@ public:
         if (static_cast<int64_t>(bytes) > cap) invalid("input " + std::to_string(id) + ": " + std::to_string(bytes) +
                                                        " bytes exceed the compiled size " + std::to_string(cap));
         if (bytes && !data) invalid("input data is null");
-        check(slhip_memcpy_h2d(mem_.at(id), data, bytes, stream_));
-        check(slhip_stream_sync(stream_));
+        const size_t slot = (bytes + 15) & ~size_t{15};
+        if (v.weight || bytes == 0 || slot > stage_.in_cap) {
+            check(slhip_memcpy_h2d(mem_.at(id), data, bytes, stream_));
+            check(slhip_stream_sync(stream_));
+            return;
+        }
+        std::lock_guard<std::mutex> lock(stage_.mu);
+        if (stage_.ran || stage_.used + slot > stage_.in_cap) {  // an earlier run's error is raised here, as by the wait above
+            stage_.ran = false;
+            stage_.used = 0;
+            check(slhip_stream_sync(stream_));
+        }
+        uint8_t* host = stage_.in + stage_.used;
+        memcpy(host, data, bytes);
+        stage_.used += slot;
+        check(stage_in(mem_.at(id), host, bytes, static_cast<hipStream_t>(stream_)));
     }
 
     void execute(int64_t T)
@@ -720,6 +736,10 @@ public:
             throw Error(SLHIP_ERR_INVALID, "Symbol 'T' = " + std::to_string(T) + " exceeds the compiled bound " +
                                                std::to_string(max_t_) + ".");
         t_ = T;
+        {
+            std::lock_guard<std::mutex> lock(stage_.mu);
+            stage_.ran = true;
+        }
         for (const Unit& u : units_) run(u, T);
     }
 
@@ -742,7 +762,15 @@ public:
         const int64_t n = v.bytes(t_);
         if (static_cast<int64_t>(bytes) != n)
             invalid("output " + std::to_string(id) + " holds " + std::to_string(n) + " bytes, destination " + std::to_string(bytes));
-        check(slhip_stream_sync(stream_));  // raises a pending gather index error
+        if (n && bytes <= stage_.out_cap) {
+            std::lock_guard<std::mutex> lock(stage_.mu);
+            stage_.ran = false;
+            stage_.used = 0;
+            check(stage_out(stage_.out, mem_.at(id), bytes, stage_.err, static_cast<hipStream_t>(stream_)));  // raises a pending gather index error
+            memcpy(data, stage_.out, bytes);
+            return;
+        }
+        check(slhip_stream_sync(stream_));
         if (n) check(slhip_memcpy_d2h(data, mem_.at(id), bytes, stream_));
         check(slhip_stream_sync(stream_));
     }
@@ -786,6 +814,18 @@ private:
     std::vector<int64_t> scratch_bytes_;  // the quantized activation copies (assign_q8)
     std::vector<void*> scratch_;
     std::map<std::string, int64_t> scalars_;
+    // Pinned memory of this segment that small inputs and outputs pass through (stage_in, stage_out), so that a step waits
+    // for the GPU once. Inputs take slots until the next wait; `ran`: units were launched since the last one.
+    struct Staging {
+        static constexpr size_t kMax = 256 * 1024;  // each way; above it the runtime's copies stream as well
+        std::mutex mu;
+        void* base = nullptr;
+        uint8_t *in = nullptr, *out = nullptr;
+        uint32_t* err = nullptr;
+        size_t in_cap = 0, out_cap = 0, used = 0;
+        bool ran = false;
+        ~Staging() { slhip_host_free(base); }
+    } stage_;
     int64_t device_bytes_ = 0;
     slhip_stream stream_ = nullptr;
 
@@ -1568,6 +1608,18 @@ private:
             scratch_.push_back(p);
             device_bytes_ += n;
         }
+        size_t in = 0, out = 0;
+        for (const auto& kv : g_.values) {
+            const size_t n = (static_cast<size_t>(std::max<int64_t>(kv.second.bytes(max_t_), 0)) + 15) & ~size_t{15};
+            if (kv.second.input && !kv.second.weight) in = std::min(in + n, Staging::kMax);
+            if (kv.second.output) out = std::max(out, std::min(n, Staging::kMax));
+        }
+        if (slhip_host_malloc(&stage_.base, in + out + 64) != SLHIP_OK) return;  // (then the runtime's copies)
+        stage_.err = static_cast<uint32_t*>(stage_.base);
+        stage_.out = static_cast<uint8_t*>(stage_.base) + 64;
+        stage_.in = stage_.out + out;
+        stage_.in_cap = in;
+        stage_.out_cap = out;
     }
 
     // The fused group's program (slhip_ew_program) on the segment's buffers.

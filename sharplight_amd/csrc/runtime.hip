@@ -136,6 +136,35 @@ static int take_device_error()
     }
 }
 
+static __global__ __launch_bounds__(256) void copy_staged(uint8_t* dst, const uint8_t* src, size_t bytes, uint32_t* err_dst, const uint32_t* err_src)
+{
+    const size_t o = (static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x) * 16;
+    if (o + 16 <= bytes)
+        *reinterpret_cast<uint4*>(dst + o) = *reinterpret_cast<const uint4*>(src + o);
+    else
+        for (size_t i = o; i < bytes; i++) dst[i] = src[i];
+    if (err_dst && blockIdx.x == 0 && threadIdx.x < 8) err_dst[threadIdx.x] = err_src[threadIdx.x];
+}
+
+static int launch_copy(void* dst, const void* src, size_t bytes, uint32_t* err_dst, const uint32_t* err_src, hipStream_t st)
+{
+    copy_staged<<<dim3(static_cast<unsigned>((bytes + 4095) / 4096)), 256, 0, st>>>(
+        static_cast<uint8_t*>(dst), static_cast<const uint8_t*>(src), bytes, err_dst, err_src);
+    return check_launch("copy_staged");
+}
+
+int stage_in(void* dst, const void* host, size_t bytes, hipStream_t st) { return launch_copy(dst, host, bytes, nullptr, nullptr, st); }
+
+int stage_out(void* host, const void* src, size_t bytes, uint32_t* host_err, hipStream_t st)
+{
+    uint32_t* w = nullptr;
+    int r = error_word(&w);
+    if (r == SLHIP_OK) r = launch_copy(host, src, bytes, host_err, w, st);
+    if (r != SLHIP_OK) return r;
+    SLHIP_CHECK_HIP(hipStreamSynchronize(st));
+    return *static_cast<volatile uint32_t*>(host_err) ? take_device_error() : SLHIP_OK;
+}
+
 }  // namespace slhip
 
 using namespace slhip;
