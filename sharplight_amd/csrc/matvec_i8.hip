@@ -24,6 +24,7 @@
 // dual form) at a time, copies its image to the wave's LDS region with 16-byte loads (narrower for rows that
 // are not 16-byte multiples) and issues the next row's loads before computing the current one; the block's TT
 // quantized activation rows are staged in LDS once. Each lane takes whole 32-value units (lane, lane + 64, ...).
+// Long rows of one and two tokens, whose images limit the waves a CU holds, are shared by two waves each.
 #include "matvec_i8.hpp"
 
 #include <stdlib.h>

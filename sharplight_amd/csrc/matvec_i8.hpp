@@ -730,20 +730,26 @@ __device__ __forceinline__ uint4 load_chunk(const char* row, int64_t off, int64_
     }
 }
 
-template <int FMT, int TT, int CH, bool DUAL, int U>
+template <int FMT, int TT, int CH, bool DUAL, int U, int KS>
 __global__ __launch_bounds__(kI8Threads) void matvec_i8(I8Args a)
 {
     extern __shared__ uint32_t smem[];
     constexpr int R = DUAL ? 2 : 1;
     const int lane = threadIdx.x & 63;
     const int wave = wave_id();
-    const int nch = static_cast<int>((a.wrow + 15) / 16);  // 16-byte chunks per row (the last may be partial)
+    // KS waves share a row, each a KS-th of it (whole blocks of the format and whole 16-byte chunks: i8_parts)
+    const int part = KS > 1 ? wave % KS : 0;
+    const int64_t wpart = a.wrow / KS;
+    const int nch = static_cast<int>((wpart + 15) / 16);   // 16-byte chunks per row (the last may be partial)
     const int rbw = nch * 4 + 4;                           // words per row image (+ a pad word group)
     uint32_t* rows = smem + wave * R * rbw;
     const int K = static_cast<int>(a.K);
     const int xrow = K + K / 2;
     uint8_t* xs = reinterpret_cast<uint8_t*>(smem + (kI8Threads / 64) * R * rbw);
-    const int nb = K / 32;  // units per row
+    const int nb = K / 32 / KS;  // units per row, or per part
+    const int xo = part * nb;    // the part's first unit
+    constexpr int RW = kI8Threads / 64 / KS;  // rows of a block at a time
+    __shared__ float red[KS > 1 ? 2 : 1][KS > 1 ? kI8Threads / 64 : 1][R * TT];
 
     // 16-byte rows: each matrix's chunks are padded to whole groups of 64, so a group of 64 chunks (one load
     // per lane) lies in one matrix and reads from a wave-uniform row base (no per-lane address arithmetic);
@@ -759,7 +765,7 @@ __global__ __launch_bounds__(kI8Threads) void matvec_i8(I8Args a)
             if constexpr (U == 16) {
                 const int r = g0 >= ncp ? 1 : 0;  // wave-uniform
                 const int w = g0 - r * ncp + lane;
-                const char* row = (r ? a.wu : a.wg) + n * a.wrow;
+                const char* row = (r ? a.wu : a.wg) + n * a.wrow + part * wpart;
                 if (w < nch) v[c] = load_nt(row + static_cast<uint32_t>(w) * 16u);
             } else {
                 int idx = g0 + lane;
@@ -792,8 +798,8 @@ __global__ __launch_bounds__(kI8Threads) void matvec_i8(I8Args a)
             store_batch(base, v);
         }
     };
-    const int64_t stride = static_cast<int64_t>(gridDim.x) * (kI8Threads / 64);
-    int64_t n = static_cast<int64_t>(blockIdx.x) * (kI8Threads / 64) + wave;
+    const int64_t stride = static_cast<int64_t>(gridDim.x) * RW;
+    int64_t n = static_cast<int64_t>(blockIdx.x) * RW + wave / KS;
     const int64_t n_first = n < a.N ? n : a.N - 1;
     uint4 v[CH];
     load_batch(n_first, 0, v);
@@ -811,7 +817,8 @@ __global__ __launch_bounds__(kI8Threads) void matvec_i8(I8Args a)
     rest(n_first, v);
     __syncthreads();
 
-    for (; n < a.N; n += stride) {  // wave-uniform
+    // (waves that share rows meet in every round: the block's first row decides for all)
+    for (int round = 0; (KS > 1 ? n - wave / KS : n) < a.N; n += stride, round ^= 1) {  // wave-uniform
         const int64_t next = n + stride;
         const bool more = next < a.N;
         if (more) load_batch(next, 0, v);
@@ -824,9 +831,9 @@ __global__ __launch_bounds__(kI8Threads) void matvec_i8(I8Args a)
             if constexpr (DUAL) uu = i8_unit<FMT>(rows + rbw, b);
 #pragma unroll
             for (int t = 0; t < TT; t++) {
-                const uint4* xp = reinterpret_cast<const uint4*>(xs + t * xrow + 32 * b);
+                const uint4* xp = reinterpret_cast<const uint4*>(xs + t * xrow + 32 * (xo + b));
                 const uint4 x0 = xp[0], x1 = xp[1];
-                const float4 sc = reinterpret_cast<const float4*>(xs + t * xrow + K)[b];
+                const float4 sc = reinterpret_cast<const float4*>(xs + t * xrow + K)[xo + b];
                 const float pg = unit_dot<FMT>(ug, x0, x1, sc);
                 ag[t] += own ? pg : 0.0f;
                 if (DUAL) {
@@ -835,9 +842,9 @@ __global__ __launch_bounds__(kI8Threads) void matvec_i8(I8Args a)
                 }
             }
         };
-        if (kSliceLds<FMT, TT> && K % 64 == 0) {  // wave-uniform; K-quants always, block formats with an even block count
+        if (kSliceLds<FMT, TT> && K % (64 * KS) == 0) {  // wave-uniform; K-quants always, block formats with an even block count
             // a 64-value slice per lane, its bytes read from the row images as words
-            const int nsl = K / 64;
+            const int nsl = K / 64 / KS;
             auto slice = [&](int sl, bool own) {
                 I8Unit g0, g1, u0, u1;
                 int j0, j1;
@@ -845,13 +852,13 @@ __global__ __launch_bounds__(kI8Threads) void matvec_i8(I8Args a)
                 if constexpr (DUAL) slice_units<FMT>(rows + rbw, sl, u0, u1, j0, j1);
 #pragma unroll
                 for (int t = 0; t < TT; t++) {
-                    const uint8_t* xt = xs + t * xrow;
+                    const uint8_t* xt = xs + t * xrow + 32 * xo;
                     const uint4 x00 = *reinterpret_cast<const uint4*>(xt + 32 * j0);
                     const uint4 x01 = *reinterpret_cast<const uint4*>(xt + 32 * j0 + 16);
                     const uint4 x10 = *reinterpret_cast<const uint4*>(xt + 32 * j1);
                     const uint4 x11 = *reinterpret_cast<const uint4*>(xt + 32 * j1 + 16);
-                    const float4 sc0 = *reinterpret_cast<const float4*>(xt + K + 16 * j0);
-                    const float4 sc1 = *reinterpret_cast<const float4*>(xt + K + 16 * j1);
+                    const float4 sc0 = *reinterpret_cast<const float4*>(xt + K - 16 * xo + 16 * j0);
+                    const float4 sc1 = *reinterpret_cast<const float4*>(xt + K - 16 * xo + 16 * j1);
                     const float pg = unit_dot<FMT>(g0, x00, x01, sc0) + unit_dot<FMT>(g1, x10, x11, sc1);
                     ag[t] += own ? pg : 0.0f;
                     if constexpr (DUAL) {
@@ -874,19 +881,42 @@ __global__ __launch_bounds__(kI8Threads) void matvec_i8(I8Args a)
                 unit(b < nb ? b : nb - 1, b < nb);
             }
         }
+        if constexpr (KS > 1) {  // the row's parts, added in order; `red` alternates, so one barrier a round
+#pragma unroll
+            for (int t = 0; t < TT; t++) {
+                ag[t] = wave_sum(ag[t]);
+                if (DUAL) au[t] = wave_sum(au[t]);
+                if (lane == 0) {
+                    red[round][wave][t] = ag[t];
+                    if (DUAL) red[round][wave][(R - 1) * TT + t] = au[t];
+                }
+            }
+            __syncthreads();
+#pragma unroll
+            for (int t = 0; t < TT; t++) {
+                ag[t] = red[round][wave - part][t];
+                if (DUAL) au[t] = red[round][wave - part][(R - 1) * TT + t];
+#pragma unroll
+                for (int i = 1; i < KS; i++) {
+                    ag[t] += red[round][wave - part + i][t];
+                    if (DUAL) au[t] += red[round][wave - part + i][(R - 1) * TT + t];
+                }
+            }
+        }
 #pragma unroll
         for (int t = 0; t < TT; t++) {
-            float out = wave_sum(ag[t]);
+            float out = KS > 1 ? ag[t] : wave_sum(ag[t]);
             if (DUAL) {
-                const float u = wave_sum(au[t]);
+                const float u = KS > 1 ? au[t] : wave_sum(au[t]);
                 const float g = out;
                 const float act = a.act == SLHIP_ACT_SILU        ? activate<SLHIP_ACT_SILU>(g)
                                   : a.act == SLHIP_ACT_GELU_TANH ? activate<SLHIP_ACT_GELU_TANH>(g)
                                                                  : activate<SLHIP_ACT_GELU_ERF>(g);
                 out = act * u;
-            } else if (a.bias) {
+            } else if (a.bias && (KS == 1 || n < a.N)) {
                 out = out + a.bias[n];
             }
+            if (KS > 1 && (part != 0 || n >= a.N)) continue;
             int64_t tok = a.t0 + t;
             tok = tok < a.T ? tok : a.T - 1;
             if (a.yt == SLHIP_F32)
@@ -944,23 +974,51 @@ inline I8Geom i8_geom(int fmt)
     }
 }
 
+// The blocks of matvec_i8 that are resident at once; 0 where the LDS is refused.
+template <int FMT, int TT, int CH, bool DUAL, int U, int KS>
+static int64_t resident_i8(size_t lds)
+{
+    auto kernel = matvec_i8<FMT, TT, CH, DUAL, U, KS>;
+    if (lds > kI8MaxLds || (lds > 65536 && hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                               static_cast<int>(lds)) != hipSuccess))
+        return 0;
+    int per_cu = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kI8Threads, lds) != hipSuccess || per_cu < 1) per_cu = 1;
+    return static_cast<int64_t>(device_cus_i8()) * per_cu;
+}
+
+template <int FMT, int TT, int CH, bool DUAL, int U, int KS>
+static int launch_i8(const I8Args& a, int64_t resident, size_t lds, hipStream_t st)
+{
+    constexpr int rows = kI8Threads / 64 / KS;
+    const int64_t blocks = (a.N + rows - 1) / rows;
+    matvec_i8<FMT, TT, CH, DUAL, U, KS><<<dim3(static_cast<unsigned>(blocks < resident ? blocks : resident)), kI8Threads, lds, st>>>(a);
+    return check_launch("matvec_i8");
+}
+
+// Whether a row splits into ks parts of whole blocks (256 values: whole 64-value slices too) and whole 16-byte chunks.
+inline bool i8_parts(const I8Args& a, int ks) { return a.K % (256 * ks) == 0 && a.wrow % (16 * ks) == 0; }
+
 template <int FMT, int TT, int CH, bool DUAL, int U>
 static int launch_i8(const I8Args& a, hipStream_t st)
 {
     const size_t lds = i8_lds(TT, a.K, a.wrow, DUAL);
-    auto kernel = matvec_i8<FMT, TT, CH, DUAL, U>;
-    if (lds > 65536) {
-        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
-                                                 hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
-        if (e != hipSuccess) return fail(SLHIP_ERR_HIP, "matvec_q8: %zu bytes of LDS refused: %s", lds, hipGetErrorString(e));
+    const int64_t one = resident_i8<FMT, TT, CH, DUAL, U, 1>(lds);
+    if (one == 0) return fail(SLHIP_ERR_HIP, "matvec_q8: %zu bytes of LDS refused", lds);
+    if constexpr (TT <= 2 && U == 16) {
+        // Two waves a row where long rows fill the LDS, so that more blocks stay on a CU: not where registers are the limit,
+        // nor from three (T = 2) or four blocks a CU on. us at T = 1, one wave / two, quantization included: Q4_K K = 14336,
+        // N = 4096 15.4 / 12.6, K = 28672, N = 8192 43.5 / 32.1; Q8_0 K = 14336, N = 4096 18.5 / 15.6, T = 2 23.1 / 19.7; Q8_0
+        // pair K = 8192, N = 28672 110 / 78. Past the line: Q4_K K = N = 8192 12.3 / 13.0, K = 4096, N = 14336 10.9 / 14.9;
+        // IQ4_NL K = N = 8192, T = 2 15.2 / 17.5. Four waves a row gained no more.
+        const int64_t cus = device_cus_i8();
+        const size_t half = i8_lds(TT, a.K, a.wrow / 2, DUAL);
+        if (one <= (TT == 1 ? 3 : 2) * cus && kI8MaxLds / lds <= static_cast<size_t>(one / cus) && i8_parts(a, 2)) {
+            const int64_t two = resident_i8<FMT, TT, CH, DUAL, U, 2>(half);
+            if (two > one) return launch_i8<FMT, TT, CH, DUAL, U, 2>(a, two, half, st);
+        }
     }
-    int per_cu = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kI8Threads, lds) != hipSuccess || per_cu < 1)
-        per_cu = 1;
-    const int64_t blocks = (a.N + kI8Threads / 64 - 1) / (kI8Threads / 64);
-    const int64_t resident = static_cast<int64_t>(device_cus_i8()) * per_cu;
-    kernel<<<dim3(static_cast<unsigned>(blocks < resident ? blocks : resident)), kI8Threads, lds, st>>>(a);
-    return check_launch("matvec_i8");
+    return launch_i8<FMT, TT, CH, DUAL, U, 1>(a, one, lds, st);
 }
 
 template <int FMT, int TT, bool DUAL>
