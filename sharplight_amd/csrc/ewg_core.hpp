@@ -10,8 +10,8 @@ namespace slhip {
 typedef float f4v __attribute__((ext_vector_type(4)));
 
 // Four values of an input of mode MODE and type DT at row r, columns c .. c + 3 (c + 3 < cols, or the
-// clamped last vector).
-template <int MODE, int DT>
+// clamped last vector). STREAM: with the streaming cache policy.
+template <int MODE, int DT, bool STREAM = false>
 __device__ __forceinline__ f4v fetch4_t(const void* data, int64_t r, int64_t c, int64_t cols)
 {
     f4v v;
@@ -26,10 +26,11 @@ __device__ __forceinline__ f4v fetch4_t(const void* data, int64_t r, int64_t c, 
     } else {
         const int64_t off = MODE == SLHIP_EWI_ROW ? c : r * cols + c;
         if constexpr (DT == SLHIP_F32) {
-            const float4 f = *reinterpret_cast<const float4*>(static_cast<const float*>(data) + off);
-            v[0] = f.x; v[1] = f.y; v[2] = f.z; v[3] = f.w;
+            const f4v* q = reinterpret_cast<const f4v*>(static_cast<const float*>(data) + off);
+            v = STREAM ? __builtin_nontemporal_load(q) : *q;
         } else {
-            const uint2 b = *reinterpret_cast<const uint2*>(static_cast<const uint16_t*>(data) + off);
+            const u32x2* q = reinterpret_cast<const u32x2*>(static_cast<const uint16_t*>(data) + off);
+            const u32x2 b = STREAM ? __builtin_nontemporal_load(q) : *q;
             if constexpr (DT == SLHIP_BF16) {
                 v[0] = bf16_lo(b.x); v[1] = bf16_hi(b.x); v[2] = bf16_lo(b.y); v[3] = bf16_hi(b.y);
             } else {
@@ -41,16 +42,22 @@ __device__ __forceinline__ f4v fetch4_t(const void* data, int64_t r, int64_t c, 
 }
 
 // Four values stored as DT at element offset off.
-template <int DT>
+template <int DT, bool STREAM = false>
 __device__ __forceinline__ void store4_t(void* p, int64_t off, f4v v)
 {
     if constexpr (DT == SLHIP_F32) {
-        *reinterpret_cast<float4*>(static_cast<float*>(p) + off) = make_float4(v[0], v[1], v[2], v[3]);
-    } else if constexpr (DT == SLHIP_BF16) {
-        *reinterpret_cast<uint2*>(static_cast<uint16_t*>(p) + off) =
-            make_uint2(f32_to_bf16_bits(v[0]) | (f32_to_bf16_bits(v[1]) << 16), f32_to_bf16_bits(v[2]) | (f32_to_bf16_bits(v[3]) << 16));
+        f4v* q = reinterpret_cast<f4v*>(static_cast<float*>(p) + off);
+        if (STREAM) __builtin_nontemporal_store(v, q);
+        else *q = v;
     } else {
-        *reinterpret_cast<uint2*>(static_cast<uint16_t*>(p) + off) = make_uint2(pack_f16x2(v[0], v[1]), pack_f16x2(v[2], v[3]));
+        u32x2 w;
+        if constexpr (DT == SLHIP_BF16)
+            w = u32x2{f32_to_bf16_bits(v[0]) | (f32_to_bf16_bits(v[1]) << 16), f32_to_bf16_bits(v[2]) | (f32_to_bf16_bits(v[3]) << 16)};
+        else
+            w = u32x2{pack_f16x2(v[0], v[1]), pack_f16x2(v[2], v[3])};
+        u32x2* q = reinterpret_cast<u32x2*>(static_cast<uint16_t*>(p) + off);
+        if (STREAM) __builtin_nontemporal_store(w, q);
+        else *q = w;
     }
 }
 

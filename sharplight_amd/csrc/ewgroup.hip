@@ -265,6 +265,29 @@ static void set_pow_special(EwgArgs& a)
 // Register values of the generated row form kept across its two passes: rows up to this many 256-value steps.
 constexpr int kJitKeepSteps = 16;
 
+// Whether a program is of the row form with its norm's operand kept in registers: it gets two kernels, ewg_jit and
+// ewg_jit_stream, which loads the full-shape inputs (each read once) and stores the norm's result with the streaming policy.
+static bool jit_streams(const EwgArgs& a)
+{
+    return (a.p.head.kind != SLHIP_EWN_NONE || a.p.tail.kind != SLHIP_EWN_NONE) && (a.cols + 255) / 256 <= kJitKeepSteps;
+}
+
+// The streaming kernel is for launches that the caches cannot hold anyway; memory-bound either way. Rows of 4096 f32, two
+// inputs, sum and norm stored, us plain / streaming: 33 MB 13.7 / 15.8, 67 MB 17.8 / 19.2, 134 MB 26.5 / 25.5, 201 MB 45.7 /
+// 35.9, 268 MB 58 / 49.6, 403 MB 90 / 75, 537 MB 108 / 91 to 103 (by process). Streaming the group's own outputs too loses (537 MB
+// 101), and so do two bodies in one kernel (105). The flat form is level everywhere.
+constexpr int64_t kJitStreamBytes = 144ll << 20;
+
+static bool jit_large(const EwgArgs& a)
+{
+    auto size = [](int dt) { return dt == SLHIP_F32 ? 4 : 2; };
+    int64_t per = a.p.tail.kind ? size(a.p.tail.dtype_y) : 0;
+    for (int i = 0; i < a.p.n_inputs; i++)
+        if (a.p.inputs[i].mode == SLHIP_EWI_FULL) per += size(a.p.inputs[i].dtype);
+    for (int k = 0; k < a.p.n_outputs; k++) per += size(a.p.outputs[k].dtype);
+    return a.rows > kJitStreamBytes / (per * a.cols);  // per > 0: a row form has a full input or an output
+}
+
 static std::string fbits(float v)
 {
     uint32_t u;
@@ -294,10 +317,17 @@ static std::string jit_source(const EwgArgs& a)
         snprintf(b, sizeof b, fmt, v...);
         s += b;
     };
+    const int nv = static_cast<int>((a.cols + 255) / 256);
+    const bool keep = nv <= kJitKeepSteps;
+    const bool once = jit_streams(a);
+    const char* end = once ? "}\nextern \"C\" __global__ __launch_bounds__(256) void ewg_jit(EwgJitArgs a) { body<false>(a); }\n"
+                             "extern \"C\" __global__ __launch_bounds__(256) void ewg_jit_stream(EwgJitArgs a) { body<true>(a); }\n"
+                           : "}\n";
     s += "#include \"ewg_core.hpp\"\nusing namespace slhip;\n";
     add("constexpr int64_t COLS = %lld;\n", static_cast<long long>(a.cols));
     auto fetch = [&](int i, const char* dst) {
-        add("    %s = fetch4_t<%s, %s>(a.in[%d], r, c, COLS);\n", dst, mode_name(p.inputs[i].mode), dt_name(p.inputs[i].dtype), i);
+        add("    %s = fetch4_t<%s, %s, %s>(a.in[%d], r, c, COLS);\n", dst, mode_name(p.inputs[i].mode), dt_name(p.inputs[i].dtype),
+            once && p.inputs[i].mode == SLHIP_EWI_FULL ? "STREAM" : "false", i);
     };
     auto ops = [&]() {
         for (int k = 0; k < p.n_ops; k++) {
@@ -313,7 +343,8 @@ static std::string jit_source(const EwgArgs& a)
         for (int j = 0; j < p.n_outputs; j++)
             add("    store4_t<%s>(a.out[%d], r * COLS + c, R%d);\n", dt_name(p.outputs[j].dtype), j, p.outputs[j].reg);
     };
-    s += "extern \"C\" __global__ __launch_bounds__(256) void ewg_jit(EwgJitArgs a)\n{\n";
+    s += once ? "template <bool STREAM>\n__device__ __forceinline__ void body(const EwgJitArgs& a)\n{\n"
+              : "extern \"C\" __global__ __launch_bounds__(256) void ewg_jit(EwgJitArgs a)\n{\n";
     s += "    f4v R0, R1, R2, R3, R4, R5, R6, R7, R8, R9, R10, R11, R12, R13, R14, R15;\n";
     if (!head && !tail) {
         const int64_t spans = (a.cols + 255) / 256;
@@ -330,11 +361,9 @@ static std::string jit_source(const EwgArgs& a)
         }
         ops();
         stores();
-        s += "}\n";
+        s += end;
         return s;
     }
-    const int nv = static_cast<int>((a.cols + 255) / 256);
-    const bool keep = nv <= kJitKeepSteps;
     s += "    const int64_t r = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);\n"
          "    if (r >= a.rows) return;\n"
          "    const int lane = threadIdx.x & 63;\n";
@@ -395,15 +424,16 @@ static std::string jit_source(const EwgArgs& a)
             add("    const f4v t = R%d;\n", nm.reg);
         }
         s += "    f4v yv;\n    for (int e = 0; e < 4; e++) yv[e] = (t[e] * scale) * wv[e];\n";
-        add("    store4_t<%s>(a.y, r * COLS + c, yv);\n", dt_name(nm.dtype_y));
+        add("    store4_t<%s, %s>(a.y, r * COLS + c, yv);\n", dt_name(nm.dtype_y), once ? "STREAM" : "false");
     }
-    s += "    }\n}\n";
+    s += "    }\n";
+    s += end;
     return s;
 }
 
 struct JitEntry {
     hipModule_t mod = nullptr;
-    hipFunction_t fn = nullptr;
+    hipFunction_t fn = nullptr, stream = nullptr;  // stream: the row form's second kernel
     bool failed = false;
 };
 static std::mutex g_jit_mu;
@@ -423,11 +453,12 @@ static hipFunction_t jit_kernel(const EwgArgs& a, bool capturing)
     if (!jit_enabled()) return nullptr;
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return nullptr;
+    auto pick = [&](const JitEntry& e) { return e.stream && jit_large(a) ? e.stream : e.fn; };
     const std::string src = jit_source(a);
     const std::string key = std::to_string(dev) + "\n" + src;
     std::lock_guard<std::mutex> lock(g_jit_mu);
     auto it = g_jit.find(key);
-    if (it != g_jit.end()) return it->second.failed ? nullptr : it->second.fn;
+    if (it != g_jit.end()) return it->second.failed ? nullptr : pick(it->second);
     // not under stream capture (loading a module is not a capturable operation): the interpreter runs this
     // launch, the kernel is made on the next uncaptured one (or ahead of time, ew_program_prepare)
     if (capturing) return nullptr;
@@ -459,12 +490,13 @@ static hipFunction_t jit_kernel(const EwgArgs& a, bool capturing)
     std::string code(n, '\0');
     hiprtcGetCode(prog, &code[0]);
     hiprtcDestroyProgram(&prog);
-    if (hipModuleLoadData(&e.mod, code.data()) != hipSuccess || hipModuleGetFunction(&e.fn, e.mod, "ewg_jit") != hipSuccess) {
+    if (hipModuleLoadData(&e.mod, code.data()) != hipSuccess || hipModuleGetFunction(&e.fn, e.mod, "ewg_jit") != hipSuccess ||
+        (jit_streams(a) && hipModuleGetFunction(&e.stream, e.mod, "ewg_jit_stream") != hipSuccess)) {
         fprintf(stderr, "sharplight_hip: loading a fused elementwise group's kernel failed; the interpreter runs it\n");
         return nullptr;
     }
     e.failed = false;
-    return e.fn;
+    return pick(e);
 }
 
 static int jit_launch(hipFunction_t fn, const EwgArgs& a, hipStream_t st)
