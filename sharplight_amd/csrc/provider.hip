@@ -697,7 +697,9 @@ public:
 
     ~Segment()
     {
-        if (stage_.base && stream_) slhip_stream_sync(stream_);
+        // (the staging memory outlives the copies from it; not slhip_stream_sync, which would take the device's error
+        // record, another segment's among it)
+        if (stage_.base && stream_) (void)hipStreamSynchronize(static_cast<hipStream_t>(stream_));
         for (auto& kv : mem_) slhip_free(kv.second);
         for (void* p : scratch_) slhip_free(p);
         if (stream_) slhip_stream_destroy(stream_);

@@ -1,6 +1,8 @@
 """The small copies of a compiled segment (through its pinned staging memory) at their edges: sizes that are no multiple of
 16 bytes, runs of other sizes than the compiled one, more inputs than the staging holds at once, inputs set again before
 and between runs, and sizes past it, which take the runtime's copies. Every result bit for bit."""
+import time
+
 import numpy as np
 import pytest
 
@@ -68,3 +70,18 @@ def test_a_runs_error_reaches_the_next_call(dev):
         seg.set_input(ids, np.array([1, 2], np.int32))
         seg.execute(2)
         assert np.array_equal(seg.get_output(y), t[[1, 2]])
+
+
+def test_closing_a_segment_keeps_the_error_of_another(dev):
+    g = provider.GraphBuilder()
+    tbl, ids = g.weight("f32", 10, 64), g.input("i32", "T")
+    y = g.output(g.gather(tbl, ids))
+    other = dev.compile(g, max_tokens=4)
+    with dev.compile(g, max_tokens=4) as seg:
+        seg.set_input(tbl, synth.normal(1, 1, (10, 64)))
+        seg.set_input(ids, np.array([1, 12], np.int32))
+        seg.execute(2)
+        time.sleep(0.2)  # the run has ended, nothing has waited for it
+        other.close()
+        with pytest.raises(IndexError, match="12"):
+            seg.get_output(y)
