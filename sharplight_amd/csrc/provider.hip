@@ -675,6 +675,25 @@ struct Unit {
     int shape_of = -1, head_node = -1, tail_node = -1, norm_reg = -1;
 };
 
+// Makes `device` the thread's current device for a scope.
+class OnDevice {
+public:
+    explicit OnDevice(int device)
+    {
+        if (hipGetDevice(&was_) == hipSuccess && was_ != device) switched_ = hipSetDevice(device) == hipSuccess;
+    }
+    ~OnDevice()
+    {
+        if (switched_) (void)hipSetDevice(was_);
+    }
+    OnDevice(const OnDevice&) = delete;
+    OnDevice& operator=(const OnDevice&) = delete;
+
+private:
+    int was_ = 0;
+    bool switched_ = false;
+};
+
 class Segment {
 public:
     // plan_only: lower the nodes into launches and stop (no stream, no device memory).
@@ -689,6 +708,7 @@ public:
         lower();
         assign_q8();
         if (plan_only) return;
+        check(slhip_get_device(&device_));
         check(slhip_stream_create(&stream_));
         allocate();
         prepare_groups();
@@ -719,6 +739,7 @@ public:
             check(slhip_stream_sync(stream_));
             return;
         }
+        const OnDevice here(device_);  // (the staging copies and the error record are the segment's device's)
         std::lock_guard<std::mutex> lock(stage_.mu);
         if (stage_.ran || stage_.used + slot > stage_.in_cap) {  // an earlier run's error is raised here, as by the wait above
             stage_.ran = false;
@@ -765,6 +786,7 @@ public:
         if (static_cast<int64_t>(bytes) != n)
             invalid("output " + std::to_string(id) + " holds " + std::to_string(n) + " bytes, destination " + std::to_string(bytes));
         if (n && bytes <= stage_.out_cap) {
+            const OnDevice here(device_);
             std::lock_guard<std::mutex> lock(stage_.mu);
             stage_.ran = false;
             stage_.used = 0;
@@ -830,6 +852,7 @@ private:
     } stage_;
     int64_t device_bytes_ = 0;
     slhip_stream stream_ = nullptr;
+    int device_ = 0;  // the device of the stream and the memory: the one current at compile
 
     std::map<int, std::vector<int>> consumers() const
     {

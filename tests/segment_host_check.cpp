@@ -231,12 +231,36 @@ void close_keeps_the_error_of_another()
     EXPECT(output(b) == SLHIP_OK);
     destroy(b);
 }
+
+// A thread whose current device is another one sets inputs and reads outputs, and stays on its device.
+void another_current_device()
+{
+    slhip_segment s = compile();
+    g_device = 1;
+    EXPECT(set_ids(s) == SLHIP_OK && g_device == 1);
+    g_device = 0;
+    EXPECT(run(s) == SLHIP_OK);
+    g_device = 1;
+    EXPECT(output(s) == SLHIP_OK && g_device == 1);
+    g_device = 0;
+    g_bad_gather = true;
+    EXPECT(run(s) == SLHIP_OK);
+    g_device = 1;
+    EXPECT(output(s) == SLHIP_ERR_INDEX && g_device == 1);
+    g_device = 0;
+    g_bad_gather = true;
+    EXPECT(run(s) == SLHIP_OK);
+    g_device = 1;
+    EXPECT(set_ids(s) == SLHIP_ERR_INDEX && g_device == 1);
+    destroy(s);
+}
 }  // namespace
 
 int main(int argc, char** argv)
 {
     const std::map<std::string, void (*)()> scenarios = {
         {"close_keeps_the_error_of_another", close_keeps_the_error_of_another},
+        {"another_current_device", another_current_device},
     };
     const auto it = scenarios.find(argc > 1 ? argv[1] : "");
     if (it == scenarios.end()) return 2;
