@@ -1639,7 +1639,10 @@ private:
             if (kv.second.input && !kv.second.weight) in = std::min(in + n, Staging::kMax);
             if (kv.second.output) out = std::max(out, std::min(n, Staging::kMax));
         }
-        if (slhip_host_malloc(&stage_.base, in + out + 64) != SLHIP_OK) return;  // (then the runtime's copies)
+        if (slhip_host_malloc(&stage_.base, in + out + 64) != SLHIP_OK) {  // then the runtime's copies
+            (void)hipGetLastError();  // (kept by the runtime; the next launch would be reported as failed)
+            return;
+        }
         stage_.err = static_cast<uint32_t*>(stage_.base);
         stage_.out = static_cast<uint8_t*>(stage_.base) + 64;
         stage_.in = stage_.out + out;

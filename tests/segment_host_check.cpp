@@ -254,6 +254,17 @@ void another_current_device()
     EXPECT(set_ids(s) == SLHIP_ERR_INDEX && g_device == 1);
     destroy(s);
 }
+
+// Without staging memory the runtime's copies are taken, and the refused allocation is no later call's error.
+void staging_memory_refused()
+{
+    g_refuse_host_malloc = true;
+    slhip_segment s = compile();
+    EXPECT(set_ids(s) == SLHIP_OK);
+    EXPECT(run(s) == SLHIP_OK);
+    EXPECT(output(s) == SLHIP_OK);
+    destroy(s);
+}
 }  // namespace
 
 int main(int argc, char** argv)
@@ -261,6 +272,7 @@ int main(int argc, char** argv)
     const std::map<std::string, void (*)()> scenarios = {
         {"close_keeps_the_error_of_another", close_keeps_the_error_of_another},
         {"another_current_device", another_current_device},
+        {"staging_memory_refused", staging_memory_refused},
     };
     const auto it = scenarios.find(argc > 1 ? argv[1] : "");
     if (it == scenarios.end()) return 2;

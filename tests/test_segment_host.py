@@ -26,7 +26,7 @@ def check(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("scenario", ["close_keeps_the_error_of_another", "another_current_device"])
+@pytest.mark.parametrize("scenario", ["close_keeps_the_error_of_another", "another_current_device", "staging_memory_refused"])
 def test_segment(check, scenario):
     r = subprocess.run([str(check), scenario], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0 and r.stdout == "ok\n", r.stdout + r.stderr
