@@ -742,9 +742,9 @@ public:
         const OnDevice here(device_);  // (the staging copies and the error record are the segment's device's)
         std::lock_guard<std::mutex> lock(stage_.mu);
         if (stage_.ran || stage_.used + slot > stage_.in_cap) {  // an earlier run's error is raised here, as by the wait above
-            stage_.ran = false;
-            stage_.used = 0;
-            check(slhip_stream_sync(stream_));
+            const int r = slhip_stream_sync(stream_);
+            stage_.waited(r);
+            check(r);
         }
         uint8_t* host = stage_.in + stage_.used;
         memcpy(host, data, bytes);
@@ -788,9 +788,9 @@ public:
         if (n && bytes <= stage_.out_cap) {
             const OnDevice here(device_);
             std::lock_guard<std::mutex> lock(stage_.mu);
-            stage_.ran = false;
-            stage_.used = 0;
-            check(stage_out(stage_.out, mem_.at(id), bytes, stage_.err, static_cast<hipStream_t>(stream_)));  // raises a pending gather index error
+            const int r = stage_out(stage_.out, mem_.at(id), bytes, stage_.err, static_cast<hipStream_t>(stream_));
+            stage_.waited(r);
+            check(r);  // raises a pending gather index error
             memcpy(data, stage_.out, bytes);
             return;
         }
@@ -848,6 +848,13 @@ private:
         uint32_t* err = nullptr;
         size_t in_cap = 0, out_cap = 0, used = 0;
         bool ran = false;
+        // After a wait that returned `status`: the slots are free unless it may have failed before the stream had ended.
+        void waited(int status)
+        {
+            if (status != SLHIP_OK && status != SLHIP_ERR_INDEX && status != SLHIP_ERR_CACHE) return;
+            ran = false;
+            used = 0;
+        }
         ~Staging() { slhip_host_free(base); }
     } stage_;
     int64_t device_bytes_ = 0;

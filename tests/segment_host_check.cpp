@@ -45,6 +45,8 @@ struct Call {
 };
 std::vector<Call> g_calls;
 std::set<Stream*> g_streams;
+std::map<void*, size_t> g_blocks;     // allocations and their bytes; g_pinned: those of host memory
+std::set<void*> g_pinned;
 
 hipError_t done(hipError_t e)
 {
@@ -130,17 +132,22 @@ hipError_t hipGetSymbolAddress(void** p, const void*)
 hipError_t hipMalloc(void** p, size_t n)
 {
     *p = aligned_alloc(256, (n + 511) / 256 * 256);
+    g_blocks[*p] = n;
     return hipSuccess;
 }
 hipError_t hipFree(void* p)
 {
+    g_blocks.erase(p);
+    g_pinned.erase(p);
     free(p);
     return hipSuccess;
 }
 hipError_t hipHostMalloc(void** p, size_t n, unsigned)
 {
     if (g_refuse_host_malloc) return done(hipErrorOutOfMemory);
-    return hipMalloc(p, n);
+    const hipError_t e = hipMalloc(p, n);
+    g_pinned.insert(*p);
+    return e;
 }
 hipError_t hipHostFree(void* p) { return hipFree(p); }
 hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned)
@@ -265,6 +272,28 @@ void staging_memory_refused()
     EXPECT(output(s) == SLHIP_OK);
     destroy(s);
 }
+
+// An input that is still to be copied stays in place when reading an output fails before it has waited.
+void failed_output_keeps_the_inputs()
+{
+    const char* add = "value 0 f32 T 64\nvalue 1 f32 T 64\nvalue 2 f32 T 64\ninput 0\ninput 1\noutput 2\nnode Add 0,1 -> 2\n";
+    slhip_segment s = nullptr;
+    EXPECT(slhip_segment_compile(add, 1, &s) == SLHIP_OK);
+    float in[2][64], y[64];
+    for (int i = 0; i < 64; i++) in[0][i] = 1.0f, in[1][i] = 2.0f;
+    EXPECT(slhip_segment_set_input(s, 0, in[0], sizeof in[0]) == SLHIP_OK);
+    EXPECT(slhip_segment_execute(s, 1) == SLHIP_OK);
+    g_refuse_copies = true;
+    EXPECT(slhip_segment_get_output(s, 2, y, sizeof y) != SLHIP_OK);
+    g_refuse_copies = false;
+    EXPECT(slhip_segment_set_input(s, 1, in[1], sizeof in[1]) == SLHIP_OK);
+    EXPECT(slhip_segment_get_output(s, 2, y, sizeof y) == SLHIP_OK);  // (runs what is queued)
+    int held = 0;  // device blocks that begin with the first input's rows
+    for (const auto& b : g_blocks)
+        if (b.second >= sizeof in[0] && memcmp(b.first, in[0], sizeof in[0]) == 0 && g_pinned.count(b.first) == 0) held++;
+    EXPECT(held == 1);
+    destroy(s);
+}
 }  // namespace
 
 int main(int argc, char** argv)
@@ -273,6 +302,7 @@ int main(int argc, char** argv)
         {"close_keeps_the_error_of_another", close_keeps_the_error_of_another},
         {"another_current_device", another_current_device},
         {"staging_memory_refused", staging_memory_refused},
+        {"failed_output_keeps_the_inputs", failed_output_keeps_the_inputs},
     };
     const auto it = scenarios.find(argc > 1 ? argv[1] : "");
     if (it == scenarios.end()) return 2;

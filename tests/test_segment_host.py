@@ -26,7 +26,8 @@ def check(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("scenario", ["close_keeps_the_error_of_another", "another_current_device", "staging_memory_refused"])
+@pytest.mark.parametrize("scenario", ["close_keeps_the_error_of_another", "another_current_device", "staging_memory_refused",
+                                      "failed_output_keeps_the_inputs"])
 def test_segment(check, scenario):
     r = subprocess.run([str(check), scenario], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0 and r.stdout == "ok\n", r.stdout + r.stderr
