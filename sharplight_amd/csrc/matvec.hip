@@ -1399,9 +1399,13 @@ template <int FMT>
 static int run_quant(MatvecArgs a, bool dual, hipStream_t st)
 {
     // Several tokens: the matrix cores; at two tokens only where the VALU kernel cannot hold both tokens' x in LDS
-    // (K = 14336, N = 4096, us, VALU / matvec_kw: Q4_K 38.6 / 22.0, Q6_K 76 / 30, Q8_0 38.9 / 25.4).
+    // (K = 14336, N = 4096, us, VALU / matvec_kw: Q4_K 38.6 / 22.0, Q6_K 76 / 30, Q8_0 38.9 / 25.4). Rows too long for the
+    // VALU kernel altogether are taken from the usual token counts on where K is a multiple of kLongK, else refused.
+    const bool long_row = quant_lds(1, a.K, a.wrow, dual) > kMaxLds;
+    constexpr int64_t kLongK = FMT == SLHIP_FMT_Q8_0 || FMT == SLHIP_FMT_Q6_K ? 512 : 1024;
     const int mt = Fmt<FMT>::K ? kq_min_tokens() : mq_min_tokens();
-    if (mt > 0 && (a.T >= mt || (a.T > 1 && quant_lds(2, a.K, a.wrow, dual) > kMaxLds))) {
+    if (mt > 0 && (long_row ? a.T >= mt && a.K % kLongK == 0
+                            : a.T >= mt || (a.T > 1 && quant_lds(2, a.K, a.wrow, dual) > kMaxLds))) {
         if constexpr (!Fmt<FMT>::K) {
             if (mq2_better(FMT, a, dual)) {
                 const int r = run_mq2_any(FMT, a, dual, st);
@@ -1418,7 +1422,7 @@ static int run_quant(MatvecArgs a, bool dual, hipStream_t st)
             return dual ? launch_kq_tile<FMT, true>(a, st) : launch_kq_tile<FMT, false>(a, st);
     }
     const int tt = a.T > 1 && quant_lds(2, a.K, a.wrow, dual) <= kMaxLds ? 2 : 1;
-    if (quant_lds(tt, a.K, a.wrow, dual) > kMaxLds)
+    if (long_row)
         return fail(SLHIP_ERR_UNSUPPORTED, "matvec: K = %lld does not fit in LDS for this format", static_cast<long long>(a.K));
     const int64_t per_lane = ((dual ? 2 : 1) * (a.wrow / 16) + 63) / 64;
     const int ch = per_lane <= 4 ? 4 : per_lane <= 8 ? 8 : per_lane <= 12 ? 12 : 16;
