@@ -1215,10 +1215,20 @@ static int run_mfma(MatvecArgs a, bool dual, hipStream_t st)
     return SLHIP_OK;
 }
 
-// Tokens from which bf16 weights take the matrix cores (SLHIP_MATVEC_MFMA_MIN_T; 0 disables): below it the
-// VALU kernel is already at the HBM rate. Measured at 14336 x 4096 (dual, us, VALU / matrix cores) at T = 2:
-// f32 x 41.6 / 44.3, bf16 x 45.1 / 40.0; at T = 3: f32 x 51.5 / 43.6.
-static int mfma_min_tokens(int xt) { return env_int("SLHIP_MATVEC_MFMA_MIN_T", xt == SLHIP_BF16 ? 2 : 3); }
+// Tokens from which bf16 and f16 weights take the matrix cores (SLHIP_MATVEC_MFMA_MIN_T; 0 disables): below it the VALU
+// kernel is already at the HBM rate. Measured with bf16 weights at 14336 x 4096 (dual, us, VALU / matrix cores) at T = 2: f32
+// x 41.6 / 44.3, bf16 x 45.1 / 40.0; at T = 3: f32 x 51.5 / 43.6. From two tokens where the VALU kernel cannot hold both
+// tokens' x at once (K = 14336, N = 4096: bf16 49.1 / 23.5, f16 50.2 / 35.6). f16 weights take two bf16 parts: pairs with f32
+// x two tokens later while the VALU kernel holds four tokens' x (dual at [4096, 4096] and [14336, 4096]: T = 3 18.7 / 19.5,
+// 49.9 / 60.4; T = 5 38.0 / 19.4, 97.9 / 63.2; one matrix T = 3 12.0 / 12.8, 34.1 / 29.7).
+template <int WT>
+static int mfma_min_tokens(const MatvecArgs& a, bool dual)
+{
+    const bool late = WT == SLHIP_F16 && dual && a.xt == SLHIP_F32 && token_tile(4, a.K) == 4;
+    const int usual = a.xt == SLHIP_BF16 || token_tile(2, a.K) < 2 ? 2 : 3;
+    const int mt = env_int("SLHIP_MATVEC_MFMA_MIN_T", usual);
+    return mt > 0 && late ? mt + 2 : mt;
+}
 
 // Whether a bf16 launch of up to 16 tokens is faster on the LDS-staged kernel above than on matvec_kw: where
 // matvec_kw's blocks no longer go round the chip once (it then pays whole further rounds). Measured at K = 4096 (us,
@@ -1238,13 +1248,8 @@ template <int WT>
 static int run_dense(MatvecArgs a, bool dual, hipStream_t st)
 {
     if constexpr (WT != SLHIP_F32) {
-        // The matrix cores from mfma_min_tokens on; f16 weights, which take two bf16 parts, a little later with f32 x
-        // (dual at [4096, 4096] and [14336, 4096], us, VALU / matvec_kw: T = 3 18.7 / 19.5, 49.9 / 60.4; T = 5 38.0 /
-        // 19.4, 97.9 / 63.2; one matrix T = 3 12.0 / 12.8, 34.1 / 29.7); and wherever the VALU kernel cannot hold
-        // two tokens' x at once (K = 14336, N = 4096, T = 2: bf16 49.1 / 23.5, f16 50.2 / 35.6).
-        const int base = mfma_min_tokens(a.xt);
-        const int mt = WT == SLHIP_F16 && dual && a.xt == SLHIP_F32 && base > 0 ? base + 2 : base;
-        if (mt > 0 && a.K % 64 == 0 && (a.T >= mt || (a.T > 1 && token_tile(a.T, a.K) < a.T))) {
+        const int mt = mfma_min_tokens<WT>(a, dual);
+        if (mt > 0 && a.K % 64 == 0 && a.T >= mt) {
             if (WT == SLHIP_BF16 && mfma_lds_better(a, dual)) return run_mfma(a, dual, st);
             const int r = run_kw(WT == SLHIP_BF16 ? SLHIP_FMT_BF16 : SLHIP_FMT_F16, a, dual, st);
             if (r != SLHIP_ERR_UNSUPPORTED) return r;
@@ -1375,13 +1380,10 @@ static int launch_kq_tile(const MatvecArgs& a, hipStream_t st)
     return check_launch("matvec_kq_tile");
 }
 
-// Tokens from which the 32-value block formats (Q4_0, Q8_0, Q4_1, Q5_0, Q5_1) take the matrix cores
-// (SLHIP_MATVEC_MQ_MIN_T; 0 disables). Measured at [14336, 4096] (dual, f32 x, us, VALU / matrix cores): Q4_0 T = 2
-// 28.1 / 44.1, T = 3 56.8 (in one pass of four) / 29.6; Q8_0 T = 2 32.5 / 46.2, T = 3 58.0 / 31.0.
-static int mq_min_tokens() { return env_int("SLHIP_MATVEC_MQ_MIN_T", 3); }
-// The same for the K-quants (SLHIP_MATVEC_KQ_MIN_T). Measured dual at [14336, 4096], f32 x (us, VALU / matrix cores):
-// Q4_K T = 2 26.8 / 31.1, T = 3 60.6 / 31.5; Q6_K T = 2 35.3 / 54.4, T = 3 94.2 / 54.6; Q3_K T = 3 78.0 / 46.8.
-static int kq_min_tokens() { return env_int("SLHIP_MATVEC_KQ_MIN_T", 3); }
+// Tokens from which the block formats take the matrix cores: three (SLHIP_MATVEC_MQ_MIN_T for the 32-value formats,
+// SLHIP_MATVEC_KQ_MIN_T for the K-quants; 0 disables). Measured dual at [14336, 4096], f32 x (us, VALU / matrix cores): Q4_0
+// T = 2 28.1 / 44.1, T = 3 56.8 (in one pass of four) / 29.6; Q8_0 T = 2 32.5 / 46.2, T = 3 58.0 / 31.0; Q4_K T = 2 26.8 /
+// 31.1, T = 3 60.6 / 31.5; Q6_K T = 2 35.3 / 54.4, T = 3 94.2 / 54.6; Q3_K T = 3 78.0 / 46.8. The exceptions are in run_quant.
 
 // matvec_mq2 (matvec_mq.hpp): the 32-value block formats at up to 16 tokens where matvec_kw's blocks go round the chip
 // more than once: pairs of more than 4096 rows, one matrix of more than 16384 (Q8_0: 8192). Measured at K = 4096, f32 x
@@ -1403,9 +1405,9 @@ static int run_quant(MatvecArgs a, bool dual, hipStream_t st)
     // VALU kernel altogether are taken from the usual token counts on where K is a multiple of kLongK, else refused.
     const bool long_row = quant_lds(1, a.K, a.wrow, dual) > kMaxLds;
     constexpr int64_t kLongK = FMT == SLHIP_FMT_Q8_0 || FMT == SLHIP_FMT_Q6_K ? 512 : 1024;
-    const int mt = Fmt<FMT>::K ? kq_min_tokens() : mq_min_tokens();
-    if (mt > 0 && (long_row ? a.T >= mt && a.K % kLongK == 0
-                            : a.T >= mt || (a.T > 1 && quant_lds(2, a.K, a.wrow, dual) > kMaxLds))) {
+    const int dflt = !long_row && quant_lds(2, a.K, a.wrow, dual) > kMaxLds ? 2 : 3;
+    const int mt = env_int(Fmt<FMT>::K ? "SLHIP_MATVEC_KQ_MIN_T" : "SLHIP_MATVEC_MQ_MIN_T", dflt);
+    if (mt > 0 && a.T >= mt && (!long_row || a.K % kLongK == 0)) {
         if constexpr (!Fmt<FMT>::K) {
             if (mq2_better(FMT, a, dual)) {
                 const int r = run_mq2_any(FMT, a, dual, st);

@@ -1,4 +1,5 @@
-"""The float-rows products of several tokens at the limits of their dispatch: rows too long for one token."""
+"""The float-rows products of several tokens at the limits of their dispatch: rows too long for one token, the switches that
+say from how many tokens on the matrix cores are taken."""
 import numpy as np
 import pytest
 
@@ -36,3 +37,20 @@ def test_long_rows_taken(device, fmt, T, K):
     y = _run(fmt, "f32", "f32", x, [raw], N, K).astype(np.float64)
     ref = x32.astype(np.float64) @ W.astype(np.float64).T
     assert np.abs(y - ref).max() <= 2.0 ** -17 * K * np.abs(W).max() * np.abs(x32).max()
+
+
+@pytest.mark.parametrize("fmt,name,K", [("bf16", "SLHIP_MATVEC_MFMA_MIN_T", 16384), ("f16", "SLHIP_MATVEC_MFMA_MIN_T", 8192),
+                                        ("q8_0", "SLHIP_MATVEC_MQ_MIN_T", 14336), ("q4_k", "SLHIP_MATVEC_KQ_MIN_T", 16384)])
+@pytest.mark.parametrize("T", [2, 5])
+def test_switches_hold_for_long_rows(device, monkeypatch, fmt, name, K, T):
+    """Below the switch's token count the VALU kernel runs, also where it holds one token's x at a time: every token's row is
+    then the one-token result, bit for bit."""
+    monkeypatch.setenv(name, "100")
+    monkeypatch.setenv("SLHIP_KQ_MFMA", "0")
+    N = 17
+    seed = _seed("switch", fmt, T, K)
+    raw, _ = _weights(fmt, N, K, seed, 1)
+    x, _ = _x("f32", T, K, seed)
+    y = _run(fmt, "f32", "f32", x, [raw], N, K)
+    for t in range(T):
+        assert np.array_equal(y[t].view(np.uint32), _run(fmt, "f32", "f32", x[t:t + 1], [raw], N, K)[0].view(np.uint32)), t
