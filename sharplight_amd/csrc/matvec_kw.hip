@@ -64,9 +64,7 @@ static KwShape kw_shape(int fmt, const MatvecArgs& a, bool dual)
     return best;
 }
 
-// y = x . W^T (or the dual form) for any number of tokens: K a multiple of 256 (block formats) or 64 (bf16, f16).
-// SLHIP_ERR_UNSUPPORTED where a launch would pass the grid's size.
-int run_kw(int fmt, const MatvecArgs& a, bool dual, hipStream_t st)
+static int run_rows(int fmt, const MatvecArgs& a, bool dual, hipStream_t st)
 {
     const KwShape s = kw_shape(fmt, a, dual);
     auto launch = [&](auto kw, auto tile) { return s.mt ? kw(fmt, a, dual, s.mt, s.tn, st) : tile(fmt, a, dual, st); };
@@ -85,6 +83,26 @@ int run_kw(int fmt, const MatvecArgs& a, bool dual, hipStream_t st)
     case SLHIP_FMT_F16: return launch(launch_kw_part5, launch_tile_part5);
     default: return SLHIP_ERR_UNSUPPORTED;
     }
+}
+
+// y = x . W^T (or the dual form) for any number of tokens: K a multiple of 256 (block formats) or 64 (bf16, f16).
+// SLHIP_ERR_UNSUPPORTED where a launch would pass the grid's size.
+int run_kw(int fmt, const MatvecArgs& a, bool dual, hipStream_t st)
+{
+    // A lane addresses its block's rows (up to 128) by 32-bit offsets: longer rows go in slices of N whose rows those reach.
+    const int64_t reach = UINT32_MAX / a.wrow > 0 ? UINT32_MAX / a.wrow : 1;
+    if (reach >= 128 || a.N <= reach) return run_rows(fmt, a, dual, st);
+    for (int64_t n = 0; n < a.N; n += reach) {
+        MatvecArgs b = a;
+        b.N = a.N - n < reach ? a.N - n : reach;
+        b.wg += n * a.wrow;
+        if (dual) b.wu += n * a.wrow;
+        b.y = static_cast<char*>(a.y) + n * (a.yt == SLHIP_F32 ? 4 : 2);
+        if (a.bias) b.bias += n;
+        const int r = run_rows(fmt, b, dual, st);
+        if (r != SLHIP_OK) return r;
+    }
+    return SLHIP_OK;
 }
 
 }  // namespace slhip

@@ -402,21 +402,21 @@ __global__ __launch_bounds__(64 * kKwWaves) __attribute__((amdgpu_waves_per_eu(2
             tok = tok < a.T ? tok : a.T - 1;
             xp[t] = static_cast<const char*>(a.x) + (tok * a.xs + 8 * g) * (XF32 ? 4 : 2);
         }
-        auto load_x = [&](int k, int b) {  // values k .. k + 31 of the tokens' rows
+        auto load_x = [&](int k, int b) {  // 32-value block k of the tokens' rows
 #pragma unroll
             for (int t = 0; t < MT; t++) {
                 if constexpr (XF32) {
-                    const float4* p = reinterpret_cast<const float4*>(xp[t] + static_cast<int64_t>(k) * 4);
+                    const float4* p = reinterpret_cast<const float4*>(xp[t] + static_cast<int64_t>(k) * 128);
                     x[b][t].f[0] = p[0];
                     x[b][t].f[1] = p[1];
                 } else {
-                    x[b][t].b = *reinterpret_cast<const uint4*>(xp[t] + static_cast<int64_t>(k) * 2);
+                    x[b][t].b = *reinterpret_cast<const uint4*>(xp[t] + static_cast<int64_t>(k) * 64);
                 }
             }
         };
         load_w(s0);
 #pragma unroll
-        for (int u = 0; u < PD; u++) load_x((s0 * SKB + u) * 32, u);
+        for (int u = 0; u < PD; u++) load_x(s0 * SKB + u, u);
 
         for (int s = s0; s < s1; s++) {
             wave_lds_sync();  // the previous stage's reads, by every lane, come first
@@ -449,7 +449,7 @@ __global__ __launch_bounds__(64 * kKwWaves) __attribute__((amdgpu_waves_per_eu(2
                 X cur[MT];
 #pragma unroll
                 for (int t = 0; t < MT; t++) cur[t] = x[u % PD][t];
-                load_x(32 * (u + PD < SKB ? s * SKB + u + PD : sn * SKB + u + PD - SKB), u % PD);
+                load_x(u + PD < SKB ? s * SKB + u + PD : sn * SKB + u + PD - SKB, u % PD);
 #pragma unroll
                 for (int t = 0; t < MT; t++) {
                     uint4 P[NP + kKwXParts<FMT>];

@@ -1,5 +1,6 @@
 """The float-rows products of several tokens at the limits of their dispatch: rows too long for one token, the switches that
-say from how many tokens on the matrix cores are taken."""
+say from how many tokens on the matrix cores are taken, and rows whose bytes or
+values pass 32 bits."""
 import numpy as np
 import pytest
 
@@ -54,3 +55,29 @@ def test_switches_hold_for_long_rows(device, monkeypatch, fmt, name, K, T):
     y = _run(fmt, "f32", "f32", x, [raw], N, K)
     for t in range(T):
         assert np.array_equal(y[t].view(np.uint32), _run(fmt, "f32", "f32", x[t:t + 1], [raw], N, K)[0].view(np.uint32)), t
+
+
+@pytest.mark.parametrize("K,N", [(512 * 526400, 16), (2 ** 31 + 1024, 1)])  # rows of 286 MB (16 of them past 2^32 bytes); values past 2^31
+def test_rows_past_32_bits(device, K, N):
+    """Q8_0 rows and x of zeros but for a few blocks, at the ends of the first and last row: the sums are those blocks'."""
+    T, wrow = 3, K // 32 * 34
+    rng = np.random.default_rng(7)
+    ref = np.zeros((T, N))
+    with Dev() as d:
+        log(f"q8_0 K={K} N={N} T={T}: {N * wrow >> 20} MiB of weights, {T * K * 2 >> 20} MiB of x")
+        pw, px, py = d.empty(N * wrow, fill=0), d.empty(T * K * 2, fill=0), d.empty(T * N * 4)
+        for b in {0, 5, K // 64, K // 32 - 1}:
+            xb = rng.integers(-8, 9, (T, 32)).astype(np.float32)
+            for t in range(T):
+                x16 = np.ascontiguousarray(xb[t].view(np.uint32) >> 16).astype(np.uint16)
+                native.call("slhip_memcpy_h2d", px + (t * K + 32 * b) * 2, x16.ctypes.data, 64, None)
+                native.synchronize()
+            for n in {0, N - 1}:
+                q = rng.integers(-127, 128, 32).astype(np.int8)
+                block = np.concatenate([np.float16([1.0]).view(np.int8), q])
+                native.call("slhip_memcpy_h2d", pw + n * wrow + 34 * b, block.ctypes.data, 34, None)
+                native.synchronize()
+                ref[:, n] += xb @ q.astype(np.float64)
+        native.matvec("q8_0", "bf16", "f32", px, T, K, pw, N, py)
+        native.synchronize()
+        assert np.array_equal(d.get(py, (T, N), np.float32), ref)
