@@ -30,15 +30,29 @@ typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ bf16x8_t as_bf16x8(const uint4& v) { return __builtin_bit_cast(bf16x8_t, v); }
 
-// split3 for finite x: the same parts without the guard.
-__device__ __forceinline__ void split3_finite(const float* x, uint4& h, uint4& m, uint4& l)
+// Two f32 as a bf16 pair without rounding: their top halves.
+__device__ __forceinline__ uint32_t top_bf16x2(float lo, float hi)
+{
+    return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u);
+}
+
+// x[0..7] (f32) as three bf16 vectors with h + m + l == x: h the top 8 significant bits, cut off and not rounded so that
+// values near the end of f32's range, which rounding would make infinite, keep a finite remainder; m the remainder's
+// nearest bf16, l the rest (at most 8 bits, so exact). GUARD: an infinite x keeps only h (inf - inf would make the remainders
+// NaN); of a NaN the remainders are NaN, whatever h has become.
+template <bool GUARD>
+__device__ __forceinline__ void split3_as(const float* x, uint4& h, uint4& m, uint4& l)
 {
     uint32_t hw[4], mw[4], lw[4];
 #pragma unroll
     for (int i = 0; i < 4; i++) {
         const float a0 = x[2 * i], a1 = x[2 * i + 1];
-        hw[i] = pack_bf16x2(a0, a1);
-        const float r0 = a0 - bf16_lo(hw[i]), r1 = a1 - bf16_hi(hw[i]);
+        hw[i] = top_bf16x2(a0, a1);
+        float r0 = a0 - bf16_hi(__float_as_uint(a0)), r1 = a1 - bf16_hi(__float_as_uint(a1));
+        if (GUARD) {
+            r0 = fabsf(a0) == __builtin_inff() ? 0.0f : r0;
+            r1 = fabsf(a1) == __builtin_inff() ? 0.0f : r1;
+        }
         mw[i] = pack_bf16x2(r0, r1);
         lw[i] = pack_bf16x2(r0 - bf16_lo(mw[i]), r1 - bf16_hi(mw[i]));
     }
@@ -47,25 +61,9 @@ __device__ __forceinline__ void split3_finite(const float* x, uint4& h, uint4& m
     l = make_uint4(lw[0], lw[1], lw[2], lw[3]);
 }
 
-// x[0..7] (f32) as three bf16 vectors with h + m + l == x; a non-finite x keeps only h (inf - inf would
-// otherwise make the remainders NaN).
-__device__ __forceinline__ void split3(const float* x, uint4& h, uint4& m, uint4& l)
-{
-    uint32_t hw[4], mw[4], lw[4];
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const float a0 = x[2 * i], a1 = x[2 * i + 1];
-        hw[i] = pack_bf16x2(a0, a1);
-        float r0 = a0 - bf16_lo(hw[i]), r1 = a1 - bf16_hi(hw[i]);
-        r0 = r0 == r0 ? r0 : 0.0f;
-        r1 = r1 == r1 ? r1 : 0.0f;
-        mw[i] = pack_bf16x2(r0, r1);
-        lw[i] = pack_bf16x2(r0 - bf16_lo(mw[i]), r1 - bf16_hi(mw[i]));
-    }
-    h = make_uint4(hw[0], hw[1], hw[2], hw[3]);
-    m = make_uint4(mw[0], mw[1], mw[2], mw[3]);
-    l = make_uint4(lw[0], lw[1], lw[2], lw[3]);
-}
+// For finite x, and for any x.
+__device__ __forceinline__ void split3_finite(const float* x, uint4& h, uint4& m, uint4& l) { split3_as<false>(x, h, m, l); }
+__device__ __forceinline__ void split3(const float* x, uint4& h, uint4& m, uint4& l) { split3_as<true>(x, h, m, l); }
 
 template <int FMT> struct MqGeom;
 // SKB: 32-value blocks per stage, RB: bytes of one row per stage, UB: bytes per staging load

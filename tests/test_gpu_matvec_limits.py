@@ -1,6 +1,6 @@
 """The float-rows products of several tokens at the limits of their dispatch: rows too long for one token, the switches that
 say from how many tokens on the matrix cores are taken, and rows whose bytes or
-values pass 32 bits."""
+values pass 32 bits, and activations at the ends of f32."""
 import numpy as np
 import pytest
 
@@ -81,3 +81,25 @@ def test_rows_past_32_bits(device, K, N):
         native.matvec("q8_0", "bf16", "f32", px, T, K, pw, N, py)
         native.synchronize()
         assert np.array_equal(d.get(py, (T, N), np.float32), ref)
+
+
+@pytest.mark.parametrize("fmt,T,K,N", [("f16", 3, 256, 40), ("f16", 19, 320, 2900), ("f16", 300, 192, 8209), ("bf16", 2, 8448, 33),
+                                       ("bf16", 16, 256, 40), ("bf16", 300, 128, 8209), ("bf16", 5, 512, 20490)])
+def test_largest_activations(device, fmt, T, K, N):
+    """x of f32's lowest and highest value (as masks have them) times weights small enough: finite sums within f32 rounding,
+    on matvec_kw and matmul_tile."""
+    big = np.finfo(np.float32).max
+    seed = _seed("largest", fmt, T, K, N)
+    raw, W = _weights(fmt, N, K, seed, 1)
+    x, _ = _x("f32", T, K, seed)
+    x = x.copy()
+    x[0, 3], x[1, K - 1], x[T - 1, 70], x[T // 2, 40] = -big, big, np.float32(3.397e38), -big
+    y = _run(fmt, "f32", "f32", x, [raw], N, K).astype(np.float64)
+    ref = x.astype(np.float64) @ W.astype(np.float64).T
+    S = np.abs(x).astype(np.float64) @ np.abs(W).astype(np.float64).T
+    fits = S < 0.99 * big
+    assert fits[[0, 1]].any()
+    bad = np.abs(y - ref)[fits] > 2.0 ** -17 * S[fits] + 1e-30
+    assert not bad.any() and np.isfinite(y[fits]).all()
+    over = np.abs(ref) > 1.01 * big
+    assert np.isinf(y[over]).all()
