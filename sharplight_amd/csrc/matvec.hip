@@ -1237,7 +1237,7 @@ static int mfma_min_tokens(const MatvecArgs& a, bool dual)
 // matrix, f32 x, N = 20480 37.8 / 36.9; 45.3 / 43.4, N = 28672 45.7 / 47.2; 59.8 / 51.7.
 static bool mfma_lds_better(const MatvecArgs& a, bool dual)
 {
-    if (a.K % 256 != 0 || a.T > 16) return false;
+    if (a.K % 256 != 0 || a.T > 16 || (a.T < 3 && a.xt == SLHIP_F32)) return false;
     return dual ? a.N > (a.xt == SLHIP_F32 ? 8192 : 4096) : a.xt != SLHIP_F32 && a.N > 16384;
 }
 

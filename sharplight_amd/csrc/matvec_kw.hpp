@@ -402,15 +402,15 @@ __global__ __launch_bounds__(64 * kKwWaves) __attribute__((amdgpu_waves_per_eu(2
             tok = tok < a.T ? tok : a.T - 1;
             xp[t] = static_cast<const char*>(a.x) + (tok * a.xs + 8 * g) * (XF32 ? 4 : 2);
         }
-        auto load_x = [&](int k, int b) {  // 32-value block k of the tokens' rows
+        auto load_x = [&](uint32_t k, int b) {  // 32-value block k of the tokens' rows (unsigned: signed, the 4 x 4 blocks spill more)
 #pragma unroll
             for (int t = 0; t < MT; t++) {
                 if constexpr (XF32) {
-                    const float4* p = reinterpret_cast<const float4*>(xp[t] + static_cast<int64_t>(k) * 128);
+                    const float4* p = reinterpret_cast<const float4*>(xp[t] + static_cast<uint64_t>(k) * 128);
                     x[b][t].f[0] = p[0];
                     x[b][t].f[1] = p[1];
                 } else {
-                    x[b][t].b = *reinterpret_cast<const uint4*>(xp[t] + static_cast<int64_t>(k) * 64);
+                    x[b][t].b = *reinterpret_cast<const uint4*>(xp[t] + static_cast<uint64_t>(k) * 64);
                 }
             }
         };
