@@ -38,7 +38,8 @@ __device__ __forceinline__ uint32_t top_bf16x2(float lo, float hi)
 
 // x[0..7] (f32) as three bf16 vectors with h + m + l == x: h the top 8 significant bits, cut off and not rounded so that
 // values near the end of f32's range, which rounding would make infinite, keep a finite remainder; m the remainder's
-// nearest bf16, l the rest (at most 8 bits, so exact). GUARD: an infinite x keeps only h (inf - inf would make the remainders
+// nearest bf16, l the rest (at most 8 bits, so exact). The remainder is taken against the packed pair, so that x's registers
+// are free of it at once. GUARD: an infinite x keeps only h (inf - inf would make the remainders
 // NaN); of a NaN the remainders are NaN, whatever h has become.
 template <bool GUARD>
 __device__ __forceinline__ void split3_as(const float* x, uint4& h, uint4& m, uint4& l)
@@ -48,7 +49,7 @@ __device__ __forceinline__ void split3_as(const float* x, uint4& h, uint4& m, ui
     for (int i = 0; i < 4; i++) {
         const float a0 = x[2 * i], a1 = x[2 * i + 1];
         hw[i] = top_bf16x2(a0, a1);
-        float r0 = a0 - bf16_hi(__float_as_uint(a0)), r1 = a1 - bf16_hi(__float_as_uint(a1));
+        float r0 = a0 - bf16_lo(hw[i]), r1 = a1 - bf16_hi(hw[i]);
         if (GUARD) {
             r0 = fabsf(a0) == __builtin_inff() ? 0.0f : r0;
             r1 = fabsf(a1) == __builtin_inff() ? 0.0f : r1;
