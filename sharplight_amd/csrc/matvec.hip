@@ -1238,7 +1238,9 @@ static int mfma_min_tokens(const MatvecArgs& a, bool dual)
 static bool mfma_lds_better(const MatvecArgs& a, bool dual)
 {
     if (a.K % 256 != 0 || a.T > 16 || (a.T < 3 && a.xt == SLHIP_F32)) return false;
-    return dual ? a.N > (a.xt == SLHIP_F32 ? 8192 : 4096) : a.xt != SLHIP_F32 && a.N > 16384;
+    if (dual) return a.N > (a.xt == SLHIP_F32 ? 8192 : 4096);
+    if (a.xt == SLHIP_F32) return false;
+    return a.N > 16384 || (a.T <= 8 && a.N > 6144 && a.K > 2048 && a.K < 8192);
 }
 
 int run_kw(int fmt, const MatvecArgs& a, bool dual, hipStream_t st);
@@ -1295,15 +1297,12 @@ static QGeom quant_geom(int fmt)
 
 constexpr size_t kMaxLds = 160 * 1024;  // gfx950 LDS per workgroup
 
-static int device_cus()
+int device_cus()
 {
-    static int cus = 0;
-    if (!cus) {
-        int dev = 0;
-        if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-            cus <= 0)
-            cus = 256;
-    }
+    static const int cus = [] {
+        int dev = 0, n = 0;
+        return hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0 ? n : 256;
+    }();
     return cus;
 }
 
@@ -1362,7 +1361,7 @@ static int quant_ch(const MatvecArgs& a, int ch, hipStream_t st)
 template <int FMT, bool DUAL>
 static int quant_tt(const MatvecArgs& a, int tt, int ch, hipStream_t st)
 {
-    return tt == 1 ? quant_ch<FMT, 1, DUAL>(a, ch, st) : quant_ch<FMT, 2, DUAL>(a, ch, st);
+    return tt == 1 ? quant_ch<FMT, 1, DUAL>(a, ch, st) : tt == 2 ? quant_ch<FMT, 2, DUAL>(a, ch, st) : quant_ch<FMT, 4, DUAL>(a, ch, st);
 }
 
 template <int FMT, bool DUAL>
@@ -1384,17 +1383,25 @@ static int launch_kq_tile(const MatvecArgs& a, hipStream_t st)
 // T = 2 28.1 / 44.1, T = 3 56.8 (in one pass of four) / 29.6; Q8_0 T = 2 32.5 / 46.2, T = 3 58.0 / 31.0; Q4_K T = 2 26.8 /
 // 31.1, T = 3 60.6 / 31.5; Q6_K T = 2 35.3 / 54.4, T = 3 94.2 / 54.6; Q3_K T = 3 78.0 / 46.8. The exceptions are in run_quant.
 
-// matvec_mq2 (matvec_mq.hpp): the 32-value block formats at up to 16 tokens where matvec_kw's blocks go round the chip
-// more than once: pairs of more than 4096 rows, one matrix of more than 16384 (Q8_0: 8192). Measured at K = 4096, f32 x
-// (us, mq2 / matvec_kw at 3 tokens; 16): pairs Q4_0 N = 4096 19.3 / 13.6; 20.1 / 15.1, N = 6144 18.8 / 19.7; 20.2 /
-// 20.3, N = 14336 29.6 / 38.2; 33.0 / 39.5; Q8_0 N = 4096 18.7 / 15.0; 20.9 / 17.0, N = 6144 19.9 / 22.3; 21.1 / 23.1,
-// N = 14336 31.0 / 45.0; 34.1 / 47.4; one matrix Q4_0 N = 14336 20.3 / 20.2; 23.6 / 20.8, N = 20480 28.4 / 35.0; 32.4 /
-// 38.1; Q8_0 N = 8192 13.4 / 14.8; 16.0 / 15.9, N = 14336 20.1 / 23.9; 24.9 / 25.1.
-int run_mq2_any(int fmt, const MatvecArgs& a, bool dual, hipStream_t st);
-static bool mq2_better(int fmt, const MatvecArgs& a, bool dual)
+int run_mq2_part0(int fmt, const MatvecArgs& a, bool dual, hipStream_t st);
+int run_mq2_part1(int fmt, const MatvecArgs& a, bool dual, hipStream_t st);
+int run_mq2_part2(int fmt, const MatvecArgs& a, bool dual, hipStream_t st);
+
+static int run_mq2_any(int fmt, const MatvecArgs& a, bool dual, hipStream_t st)
 {
-    return a.T <= 16 && a.N > (dual ? 4096 : fmt == SLHIP_FMT_Q8_0 ? 8192 : 16384);
+    switch (fmt) {
+    case SLHIP_FMT_Q4_0:
+    case SLHIP_FMT_Q8_0:
+    case SLHIP_FMT_Q4_1:
+    case SLHIP_FMT_Q5_0:
+    case SLHIP_FMT_Q5_1: return run_mq2_part0(fmt, a, dual, st);
+    case SLHIP_FMT_Q4_K:
+    case SLHIP_FMT_Q5_K: return run_mq2_part1(fmt, a, dual, st);
+    default: return run_mq2_part2(fmt, a, dual, st);
+    }
 }
+
+bool mq2_better(int fmt, const MatvecArgs& a, bool dual);
 
 template <int FMT>
 static int run_quant(MatvecArgs a, bool dual, hipStream_t st)
@@ -1406,12 +1413,14 @@ static int run_quant(MatvecArgs a, bool dual, hipStream_t st)
     constexpr int64_t kLongK = FMT == SLHIP_FMT_Q8_0 || FMT == SLHIP_FMT_Q6_K ? 512 : 1024;
     const int dflt = !long_row && quant_lds(2, a.K, a.wrow, dual) > kMaxLds ? 2 : 3;
     const int mt = env_int(Fmt<FMT>::K ? "SLHIP_MATVEC_KQ_MIN_T" : "SLHIP_MATVEC_MQ_MIN_T", dflt);
-    if (mt > 0 && a.T >= mt && (!long_row || a.K % kLongK == 0)) {
-        if constexpr (!Fmt<FMT>::K) {
-            if (mq2_better(FMT, a, dual)) {
-                const int r = run_mq2_any(FMT, a, dual, st);
-                if (r != SLHIP_ERR_UNSUPPORTED) return r;
-            }
+    // Few rows at three and four tokens: one pass of four on the VALU kernel where K is off matvec_mq2's stages and so an
+    // uneven split for matvec_kw, too (K = 2560, N = 1024, T = 3, us, matvec_kw / VALU: Q4_0 9.6 / 7.0, pair 12.0 / 7.9; Q4_K
+    // 8.7 / 7.0; Q5_0 pair 14.5 / 8.6; N = 2048 pair 12.8 / 10.0; N = 4096 level).
+    const bool four = a.K % kLongK != 0 && a.N <= 2048 && a.T <= 4 && quant_lds(4, a.K, a.wrow, dual) <= kMaxLds;
+    if (mt > 0 && a.T >= mt && !(four && a.T > 2) && (!long_row || a.K % kLongK == 0)) {
+        if (mq2_better(FMT, a, dual)) {
+            const int r = run_mq2_any(FMT, a, dual, st);
+            if (r != SLHIP_ERR_UNSUPPORTED) return r;
         }
         const int r = run_kw(FMT, a, dual, st);
         if (r != SLHIP_ERR_UNSUPPORTED) return r;
@@ -1422,7 +1431,7 @@ static int run_quant(MatvecArgs a, bool dual, hipStream_t st)
             env_int("SLHIP_KQ_MFMA", 1))
             return dual ? launch_kq_tile<FMT, true>(a, st) : launch_kq_tile<FMT, false>(a, st);
     }
-    const int tt = a.T > 1 && quant_lds(2, a.K, a.wrow, dual) <= kMaxLds ? 2 : 1;
+    const int tt = four && a.T > 2 ? 4 : a.T > 1 && quant_lds(2, a.K, a.wrow, dual) <= kMaxLds ? 2 : 1;
     if (long_row)
         return fail(SLHIP_ERR_UNSUPPORTED, "matvec: K = %lld does not fit in LDS for this format", static_cast<long long>(a.K));
     const int64_t per_lane = ((dual ? 2 : 1) * (a.wrow / 16) + 63) / 64;

@@ -167,7 +167,7 @@ __device__ __forceinline__ uint4 kw_codes1(const uint8_t* row, int u, int g, flo
         const uint32_t sh = 4 * static_cast<uint32_t>(g >> 1);
         return nibbles_bf16((w[0] >> sh) & 0x0F0F0F0Fu, (w[1] >> sh) & 0x0F0F0F0Fu);
     } else if constexpr (FMT == SLHIP_FMT_Q5_K) {
-        return q5k_codes(row, u, g);
+        return q4k_codes<true>(row, 0, u, g);
     } else if constexpr (FMT == SLHIP_FMT_Q6_K) {
         return q6k_codes(row, 0, u, g);
     } else if constexpr (FMT == SLHIP_FMT_Q2_K || FMT == SLHIP_FMT_Q3_K) {

@@ -1,8 +1,8 @@
 #pragma once
-// The several-token (dual) matvec on the 32-value GGUF block formats with f32 or bf16 activations (the float-rows
+// The several-token (dual) matvec on GGUF block-format weights with f32 or bf16 activations (the float-rows
 // numerics: the MatMul carries f32_activations, or its row count is outside the integer-dot rule), on the bf16
-// matrix cores: matvec_mq2, for many rows and up to 16 tokens (fewer rows, more tokens and the K-quants take
-// matvec_kw, matvec_kw.hpp).
+// matrix cores: matvec_mq2, at few tokens where the dispatch (mq2_better, matvec_kw.hip) finds it ahead of matvec_kw
+// (matvec_kw.hpp), which takes the rest.
 //
 // A block of 8 waves takes a 16-row tile (a gate/up pair of tiles) and 16 tokens. Stages of SKB 32-value
 // blocks of the tile's rows move HBM -> LDS by global_load_lds (double-buffered; one vmcnt(0) ahead of the
@@ -10,9 +10,11 @@
 // v_mfma_f32_16x16x32_bf16 multiplies the tokens' x (A: lane l holds token l % 16, values 8 (l / 16) .. + 7;
 // f32 x as three bf16 parts h + m + l == x exactly, bf16 x as is) with the block's codes as exact bf16 (B:
 // lane l holds row l % 16, the same values), so lane l's sums are tokens 4 (l / 16) + i of row l % 16: each
-// lane decodes its own row's block scale once and scales with one fma per output. The
-// block minimum terms (Q4_1 / Q5_1 +m sum(x)) of a wave's 4 blocks are a 16 x 16 x 4 product (tokens x blocks .
-// blocks x rows): one v_mfma_f32_16x16x4f32 per matrix per stage. The waves' partial sums meet in LDS at the end.
+// lane decodes its own row's block scale once and scales with one fma per output. Q6_K, whose blocks hold
+// two 16-value scale groups, takes two chains, the other half's codes masked to zero; Q2_K's and Q3_K's group scales
+// are folded into the codes. The block minimum terms (Q4_K / Q5_K -dmin mn sum(x), Q4_1 / Q5_1 +m sum(x), Q2_K -dmin m per half) of a wave's
+// 4 blocks are a 16 x 16 x 4 product (tokens x blocks . blocks x rows): one v_mfma_f32_16x16x4f32 per matrix
+// (two for Q2_K's halves) per stage. The waves' partial sums meet in LDS at the end.
 //
 // Arithmetic against the reference (MatMulOp's f32 dot of dequantized rows): every product code x part is
 // exact and the sums are f32, so the result is the f32 evaluation of sum(scale * code * x) + min terms in
@@ -24,18 +26,64 @@ namespace slhip {
 
 constexpr int kMq2Waves = 8;
 
-// 32-value blocks per stage: the block formats' stage of matvec_mfma_q, halved for f32 x when that stage holds
-// 32 blocks (the x of the next stage waits in registers: 8 f32 per block and lane, two sets).
+// The multipliers of block sj (32 values) of a row image, for the value halves (a0: values 0..15, a1:
+// 16..31; equal for the 32-value scale formats), and its minimum coefficients per half (m0, m1; the min term
+// is m * sum(x) over the half, or over the whole block with m0 when the format has one minimum per block).
+// row: the row's stage bytes; sbo: the K-quant super-block's first byte in it; off: a 32-value block's first
+// byte. Layouts of Quant.cs:242-405 and Quant.KQuants.cs (ggml's).
+template <int FMT>
+__device__ __forceinline__ void mq2_scales(const uint8_t* row, int sbo, int sj, int off, float& a0, float& a1, float& m0,
+                                           float& m1)
+{
+    auto h16 = [&](int o) { return static_cast<float>(*reinterpret_cast<const _Float16*>(row + o)); };
+    auto u16 = [&](int o) { return static_cast<uint32_t>(*reinterpret_cast<const uint16_t*>(row + o)); };
+    m0 = m1 = 0.0f;
+    if constexpr (FMT == SLHIP_FMT_Q4_K || FMT == SLHIP_FMT_Q5_K) {
+        const uint32_t* w = reinterpret_cast<const uint32_t*>(row + sbo);  // 16-byte aligned super-block
+        const uint32_t hx = w[0], hy = w[1], hz = w[2], hw = w[3];
+        const int j = sj & 3, sh = 8 * j;
+        uint32_t sc, mn;
+        if (sj < 4) {
+            sc = (hy >> sh) & 63u;
+            mn = (hz >> sh) & 63u;
+        } else {
+            sc = ((hw >> sh) & 0xFu) | (((hy >> sh) >> 6 & 3u) << 4);
+            mn = (((hw >> sh) >> 4) & 0xFu) | (((hz >> sh) >> 6 & 3u) << 4);
+        }
+        a0 = a1 = __fmul_rn(f16_lo(hx), static_cast<float>(sc));
+        m0 = -__fmul_rn(f16_hi(hx), static_cast<float>(mn));
+    } else if constexpr (FMT == SLHIP_FMT_Q6_K) {
+        const float d = h16(sbo + 208);
+        const uint32_t s = u16(sbo + 192 + 2 * sj);
+        a0 = __fmul_rn(d, static_cast<float>(static_cast<int8_t>(s & 0xFFu)));
+        a1 = __fmul_rn(d, static_cast<float>(static_cast<int8_t>(s >> 8)));
+    } else if constexpr (FMT == SLHIP_FMT_Q2_K) {
+        const float dm = h16(sbo + 82);
+        const uint32_t v = u16(sbo + 2 * sj);
+        a0 = a1 = 1.0f;  // (in the codes)
+        m0 = -__fmul_rn(dm, static_cast<float>((v >> 4) & 0xFu));
+        m1 = -__fmul_rn(dm, static_cast<float>(v >> 12));
+    } else {
+        a0 = a1 = h16(off);
+        if constexpr (Fmt<FMT>::M) m0 = h16(off + 2);  // Q4_1, Q5_1: + m sum(x)
+    }
+}
+
+// The codes of block sj (32 values) of a row image, lane group g's eight (values 8g .. 8g + 7), as exact bf16.
+template <int FMT>
+__device__ __forceinline__ uint4 mq2_codes(const uint8_t* row, int sbo, int sj, int off, int g)
+{
+    if constexpr (FMT == SLHIP_FMT_Q4_K || FMT == SLHIP_FMT_Q5_K) return q4k_codes<FMT == SLHIP_FMT_Q5_K>(row, sbo, sj, g);
+    else if constexpr (FMT == SLHIP_FMT_Q6_K) return q6k_codes(row, sbo, sj, g);
+    else return mq_codes<FMT>(row, off, g);
+}
+
+// 32-value blocks per stage: MqGeom's, halved for f32 x when that stage holds 32 blocks (the x of the next stage waits in registers: 8 f32 per block and lane, two sets).
 template <int FMT, bool XF32>
 constexpr int mq2_blocks()
 {
     return XF32 && MqGeom<FMT>::SKB == 32 ? 16 : MqGeom<FMT>::SKB;
 }
-
-// 16-row tiles per block with f32 x: two, so that each block splits x into its three bf16 parts (and reads it) once
-// for 32 rows -- [14336, 4096] pairs at 16 tokens, µs: Q4_0 51 -> 40, Q8_0 56 -> 45, Q4_1 52 -> 37, Q5_0 59 -> 51,
-// Q5_1 55 -> 46.
-constexpr int kMq2Tiles = 2;
 
 template <int FMT, bool DUAL, bool XF32, int TN>
 __global__ __launch_bounds__(64 * kMq2Waves) __attribute__((amdgpu_waves_per_eu(TN == 2 ? 4 : 1))) void matvec_mq2(MatvecArgs a)
@@ -52,7 +100,13 @@ __global__ __launch_bounds__(64 * kMq2Waves) __attribute__((amdgpu_waves_per_eu(
     constexpr int NT = 64 * kMq2Waves;
     constexpr int LPT = (SLOTS + NT - 1) / NT;
     constexpr int BPW = SKB / kMq2Waves;  // blocks per wave and stage
-    constexpr bool MIN = Fmt<FMT>::M;  // minimum terms
+    constexpr bool KQ = FMT == SLHIP_FMT_Q4_K || FMT == SLHIP_FMT_Q5_K;
+    constexpr bool K6 = FMT == SLHIP_FMT_Q6_K;  // two multipliers a block
+    constexpr bool Q2K = FMT == SLHIP_FMT_Q2_K;
+    // Q2_K / Q3_K: the 16-value groups' scales folded into the codes (one MFMA chain per block, not two)
+    constexpr bool FOLD = FMT == SLHIP_FMT_Q2_K || FMT == SLHIP_FMT_Q3_K;
+    constexpr bool MIN = KQ || (Fmt<FMT>::M && !Fmt<FMT>::K) || Q2K;  // minimum terms
+    constexpr int SBB = Fmt<FMT>::BB;
     constexpr int NP = XF32 ? 3 : 1;  // bf16 parts of x
     static_assert(RB % UB == 0 && SKB % kMq2Waves == 0, "stage shape");
     static_assert(!MIN || BPW <= 4, "the minimum terms take the wave's blocks as one 16 x 16 x 4 product");
@@ -121,11 +175,13 @@ __global__ __launch_bounds__(64 * kMq2Waves) __attribute__((amdgpu_waves_per_eu(
     for (int m = 0; m < G; m++) acc[m] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
 
     auto compute = [&](int b, const Xs& x) {
-        float xs0[BPW];     // the token's x sums of each block
-        float mn0[G][BPW];  // the row's minimum coefficients of each block
+        const int sbo = Fmt<FMT>::K ? ((wave * BPW) >> 3) * SBB : 0;
+        float xs0[BPW], xs1[BPW];  // the token's x sums of each block (Q2_K: of each half)
+        float mn0[G][BPW], mn1[G][BPW];  // the row's minimum coefficients of each block
 #pragma unroll
         for (int j = 0; j < BPW; j++) {
             const int blk = wave * BPW + j;
+            const int sj = blk & 7;  // K-quant 32-value block in its super-block
             const int off = blk * Fmt<FMT>::BB;
             uint4 P[NP];
             float v[8];
@@ -145,23 +201,65 @@ __global__ __launch_bounds__(64 * kMq2Waves) __attribute__((amdgpu_waves_per_eu(
             }
             if constexpr (MIN) {
                 float ps = ps8;
-                ps += __shfl_xor(ps, 16);
-                ps += __shfl_xor(ps, 32);
-                xs0[j] = ps;
+                if constexpr (Q2K) {  // per 16-value half: lane groups {0, 1} and {2, 3}
+                    const float p01 = ps + __shfl_xor(ps, 16);
+                    const float other = __shfl_xor(p01, 32);
+                    xs0[j] = g < 2 ? p01 : other;
+                    xs1[j] = g < 2 ? other : p01;
+                } else {
+                    ps += __shfl_xor(ps, 16);
+                    ps += __shfl_xor(ps, 32);
+                    xs0[j] = ps;
+                }
             }
 #pragma unroll
             for (int m = 0; m < G; m++) {
                 const uint8_t* rw = rowp(b, m, r);
-                const uint4 C = mq_codes<FMT>(rw, off, g);
-                auto h16 = [&](int o) { return static_cast<float>(*reinterpret_cast<const _Float16*>(rw + o)); };
-                const float a0 = h16(off);
-                if constexpr (MIN) mn0[m][j] = h16(off + 2);
-                f32x4_t c = {0.0f, 0.0f, 0.0f, 0.0f};
+                const f32x4_t z = {0.0f, 0.0f, 0.0f, 0.0f};
+                if constexpr (FOLD) {
+                    float d;
+                    const uint4 C = q23k_codes_scaled<FMT == SLHIP_FMT_Q3_K>(rw, sbo, sj, g, d);
+                    if constexpr (MIN) {
+                        float a0, a1, m0, m1;
+                        mq2_scales<FMT>(rw, sbo, sj, off, a0, a1, m0, m1);
+                        mn0[m][j] = m0;
+                        mn1[m][j] = m1;
+                    }
+                    f32x4_t c = z;
 #pragma unroll
-                for (int p = 0; p < NP; p++)
-                    c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(P[p]), as_bf16x8(C), c, 0, 0, 0);
+                    for (int p = 0; p < NP; p++)
+                        c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(P[p]), as_bf16x8(C), c, 0, 0, 0);
 #pragma unroll
-                for (int i = 0; i < 4; i++) acc[m][i] = fmaf(a0, c[i], acc[m][i]);
+                    for (int i = 0; i < 4; i++) acc[m][i] = fmaf(d, c[i], acc[m][i]);
+                } else {
+                    const uint4 C = mq2_codes<FMT>(rw, sbo, sj, off, g);
+                    float a0, a1, m0, m1;
+                    mq2_scales<FMT>(rw, sbo, sj, off, a0, a1, m0, m1);
+                    if constexpr (MIN) {
+                        mn0[m][j] = m0;
+                        mn1[m][j] = m1;
+                    }
+                    if constexpr (K6) {
+                        const uint32_t keep = g < 2 ? ~0u : 0u;
+                        const uint4 C0 = make_uint4(C.x & keep, C.y & keep, C.z & keep, C.w & keep);
+                        const uint4 C1 = make_uint4(C.x & ~keep, C.y & ~keep, C.z & ~keep, C.w & ~keep);
+                        f32x4_t c0 = z, c1 = z;
+#pragma unroll
+                        for (int p = 0; p < NP; p++) {
+                            c0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(P[p]), as_bf16x8(C0), c0, 0, 0, 0);
+                            c1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(P[p]), as_bf16x8(C1), c1, 0, 0, 0);
+                        }
+#pragma unroll
+                        for (int i = 0; i < 4; i++) acc[m][i] = fmaf(a1, c1[i], fmaf(a0, c0[i], acc[m][i]));
+                    } else {
+                        f32x4_t c = z;
+#pragma unroll
+                        for (int p = 0; p < NP; p++)
+                            c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(P[p]), as_bf16x8(C), c, 0, 0, 0);
+#pragma unroll
+                        for (int i = 0; i < 4; i++) acc[m][i] = fmaf(a0, c[i], acc[m][i]);
+                    }
+                }
             }
         }
         if constexpr (MIN) {
@@ -176,7 +274,10 @@ __global__ __launch_bounds__(64 * kMq2Waves) __attribute__((amdgpu_waves_per_eu(
             };
             const float xa = pick(xs0);
 #pragma unroll
-            for (int m = 0; m < G; m++) acc[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(xa, pick(mn0[m]), acc[m], 0, 0, 0);
+            for (int m = 0; m < G; m++) {
+                acc[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(xa, pick(mn0[m]), acc[m], 0, 0, 0);
+                if constexpr (Q2K) acc[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(pick(xs1), pick(mn1[m]), acc[m], 0, 0, 0);
+            }
         }
     };
 
@@ -254,24 +355,34 @@ inline bool mq2_fits(const MatvecArgs& a)
     return a.xt == SLHIP_F32 ? mq2_fits_x<FMT, true>(a) : mq2_fits_x<FMT, false>(a);
 }
 
-template <int FMT>
-int run_mq2(MatvecArgs a, bool dual, hipStream_t st)
+template <int FMT, bool DUAL>
+int run_mq2_form(MatvecArgs a, hipStream_t st)
 {
-    constexpr int TN = kMq2Tiles;
-    const dim3 grid1(static_cast<unsigned>((a.N + 15) / 16)), gridx(static_cast<unsigned>((a.N + 16 * TN - 1) / (16 * TN)));
+    constexpr bool no_f32 = !DUAL && FMT == SLHIP_FMT_Q4_K;  // loses to matvec_kw at every size measured
+    constexpr int TN = mq2_row_tiles(FMT, SLHIP_F32);
+    if ((a.xt == SLHIP_F32 && no_f32) || !mq2_fits<FMT>(a)) return SLHIP_ERR_UNSUPPORTED;
     for (int64_t t0 = 0; t0 < a.T; t0 += 16) {
         a.t0 = t0;
-        if (a.xt == SLHIP_F32) {
-            if (dual) matvec_mq2<FMT, true, true, TN><<<gridx, 64 * kMq2Waves, 0, st>>>(a);
-            else matvec_mq2<FMT, false, true, TN><<<gridx, 64 * kMq2Waves, 0, st>>>(a);
-        } else {
-            if (dual) matvec_mq2<FMT, true, false, 1><<<grid1, 64 * kMq2Waves, 0, st>>>(a);
-            else matvec_mq2<FMT, false, false, 1><<<grid1, 64 * kMq2Waves, 0, st>>>(a);
-        }
+        if (a.xt != SLHIP_F32)
+            matvec_mq2<FMT, DUAL, false, 1><<<dim3(static_cast<unsigned>((a.N + 15) / 16)), 64 * kMq2Waves, 0, st>>>(a);
+        else if constexpr (!no_f32)
+            matvec_mq2<FMT, DUAL, true, TN><<<dim3(static_cast<unsigned>((a.N + 16 * TN - 1) / (16 * TN))), 64 * kMq2Waves, 0, st>>>(a);
         const int r = check_launch("matvec_mq2");
         if (r != SLHIP_OK) return r;
     }
     return SLHIP_OK;
 }
+
+template <int FMT>
+int run_mq2(const MatvecArgs& a, bool dual, hipStream_t st)
+{
+    return dual ? run_mq2_form<FMT, true>(a, st) : run_mq2_form<FMT, false>(a, st);
+}
+
+// instantiated in matvec_mq_*.hip, one group of formats per unit; SLHIP_ERR_UNSUPPORTED when the launch does
+// not fit (the caller then takes matvec_kw)
+int run_mq2_part0(int fmt, const MatvecArgs& a, bool dual, hipStream_t st);
+int run_mq2_part1(int fmt, const MatvecArgs& a, bool dual, hipStream_t st);
+int run_mq2_part2(int fmt, const MatvecArgs& a, bool dual, hipStream_t st);
 
 }  // namespace slhip

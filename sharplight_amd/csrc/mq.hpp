@@ -66,13 +66,31 @@ __device__ __forceinline__ void split3_as(const float* x, uint4& h, uint4& m, ui
 __device__ __forceinline__ void split3_finite(const float* x, uint4& h, uint4& m, uint4& l) { split3_as<false>(x, h, m, l); }
 __device__ __forceinline__ void split3(const float* x, uint4& h, uint4& m, uint4& l) { split3_as<true>(x, h, m, l); }
 
+// Compute units of the device (matvec.hip).
+int device_cus();
+
+// 16-row tiles per block of matvec_mq2 (matvec_mq.hpp). With f32 x two for the 32-value block formats, so that each block
+// splits x into its three bf16 parts (and reads it) once for 32 rows -- [14336, 4096] pairs at 16 tokens, us: Q4_0 51 -> 40,
+// Q8_0 56 -> 45, Q4_1 52 -> 37, Q5_0 59 -> 51, Q5_1 55 -> 46; and for Q2_K / Q3_K with their group scales folded into the
+// codes (Q2_K 52.7 -> 48.3, Q3_K 58.0 -> 56.7); one for Q4_K / Q5_K / Q6_K, whose extra decode state then spills (Q4_K
+// 52 -> 55, Q6_K 70 -> 102).
+constexpr int mq2_row_tiles(int fmt, int xt)
+{
+    return xt == SLHIP_F32 && fmt != SLHIP_FMT_Q4_K && fmt != SLHIP_FMT_Q5_K && fmt != SLHIP_FMT_Q6_K ? 2 : 1;
+}
+
 template <int FMT> struct MqGeom;
-// SKB: 32-value blocks per stage, RB: bytes of one row per stage, UB: bytes per staging load
-template <> struct MqGeom<SLHIP_FMT_Q4_0> { static constexpr int SKB = 32, RB = 32 * 18, UB = 16; };
-template <> struct MqGeom<SLHIP_FMT_Q8_0> { static constexpr int SKB = 16, RB = 16 * 34, UB = 16; };
-template <> struct MqGeom<SLHIP_FMT_Q4_1> { static constexpr int SKB = 32, RB = 32 * 20, UB = 16; };
-template <> struct MqGeom<SLHIP_FMT_Q5_0> { static constexpr int SKB = 32, RB = 32 * 22, UB = 16; };
-template <> struct MqGeom<SLHIP_FMT_Q5_1> { static constexpr int SKB = 32, RB = 32 * 24, UB = 16; };
+// SKB: 32-value blocks per stage of matvec_mq2, RB: bytes of one row per stage
+template <> struct MqGeom<SLHIP_FMT_Q4_0> { static constexpr int SKB = 32, RB = 32 * 18; };
+template <> struct MqGeom<SLHIP_FMT_Q8_0> { static constexpr int SKB = 16, RB = 16 * 34; };
+template <> struct MqGeom<SLHIP_FMT_Q4_1> { static constexpr int SKB = 32, RB = 32 * 20; };
+template <> struct MqGeom<SLHIP_FMT_Q5_0> { static constexpr int SKB = 32, RB = 32 * 22; };
+template <> struct MqGeom<SLHIP_FMT_Q5_1> { static constexpr int SKB = 32, RB = 32 * 24; };
+template <> struct MqGeom<SLHIP_FMT_Q4_K> { static constexpr int SKB = 32, RB = 4 * 144; };  // 4 super-blocks
+template <> struct MqGeom<SLHIP_FMT_Q5_K> { static constexpr int SKB = 32, RB = 4 * 176; };
+template <> struct MqGeom<SLHIP_FMT_Q6_K> { static constexpr int SKB = 16, RB = 2 * 210; };   // 420 bytes
+template <> struct MqGeom<SLHIP_FMT_Q2_K> { static constexpr int SKB = 32, RB = 4 * 84; };    // 336 bytes
+template <> struct MqGeom<SLHIP_FMT_Q3_K> { static constexpr int SKB = 32, RB = 4 * 110; };   // 440 bytes
 
 // Eight codes of lane group g (values 8g .. 8g + 7 of the block) as four bf16 pairs, the format's offset
 // applied (Q4_0 q - 8, Q5_0 q - 16: exact); row: the row's stage bytes (4-byte aligned), off: the block's
@@ -129,16 +147,22 @@ __device__ __forceinline__ uint4 mq_codes(const uint8_t* row, int off, int g)
     return make_uint4(pack_bf16x2(f[0], f[1]), pack_bf16x2(f[2], f[3]), pack_bf16x2(f[4], f[5]), pack_bf16x2(f[6], f[7]));
 }
 
-// Eight Q5_K codes of lane group g (values 8g .. 8g + 7 of sub-block j of the super-block at `row`, 16-byte aligned) as
-// four bf16 pairs: the low (j even) or high nibbles of bytes 32 (j / 2) + 8g .. of the 128 code bytes at 48, plus 16
-// when bit j of byte l of the 32-byte qh at 16 is set (ggml's Q5_K layout).
-__device__ __forceinline__ uint4 q5k_codes(const uint8_t* row, int j, int g)
+// Eight Q4_K codes of lane group g (values 8g .. 8g + 7 of sub-block j: the low (j even) or high nibbles of
+// bytes 32 (j / 2) + 8g .. of the super-block's 128 code bytes, Quant.cs:518-545) as four bf16 pairs; sbo: the
+// super-block's first byte in the staged row (a multiple of 16), so the eight bytes are one aligned 8-byte read.
+// Q5_K (FIVE): the codes after a 32-byte qh at byte 16, and value l of sub-block j adds 16 when bit j of qh[l]
+// is set (ggml's Q5_K layout, the same scale packing as Q4_K).
+template <bool FIVE = false>
+__device__ __forceinline__ uint4 q4k_codes(const uint8_t* row, int sbo, int j, int g)
 {
-    const uint2 w = *reinterpret_cast<const uint2*>(row + 48 + 32 * (j >> 1) + 8 * g);
-    const uint2 h = *reinterpret_cast<const uint2*>(row + 16 + 8 * g);
+    const uint2 w = *reinterpret_cast<const uint2*>(row + sbo + (FIVE ? 48 : 16) + 32 * (j >> 1) + 8 * g);
     const uint32_t sh = 4 * static_cast<uint32_t>(j & 1);
-    const uint32_t lo = ((w.x >> sh) & 0x0F0F0F0Fu) | (((h.x >> j) & 0x01010101u) << 4);
-    const uint32_t hi = ((w.y >> sh) & 0x0F0F0F0Fu) | (((h.y >> j) & 0x01010101u) << 4);
+    uint32_t lo = (w.x >> sh) & 0x0F0F0F0Fu, hi = (w.y >> sh) & 0x0F0F0F0Fu;
+    if constexpr (FIVE) {
+        const uint2 h = *reinterpret_cast<const uint2*>(row + sbo + 16 + 8 * g);
+        lo |= ((h.x >> j) & 0x01010101u) << 4;
+        hi |= ((h.y >> j) & 0x01010101u) << 4;
+    }
     float f[8];
 #pragma unroll
     for (int e = 0; e < 4; e++) {
