@@ -1201,40 +1201,41 @@ static int mfma_tiles(int64_t T, int xt)
     return nt == 1 || nt == 2 ? nt : (xt == SLHIP_F32 && T > 12 ? 2 : 1);
 }
 
-static int run_mfma(MatvecArgs a, bool dual, hipStream_t st)
+static int run_mfma(MatvecArgs a, bool dual, hipStream_t st)  // up to 16 tokens
 {
     const int sk = mfma_stage(), nt = mfma_tiles(a.T, a.xt);
-    for (int64_t t0 = 0; t0 < a.T; t0 += 16) {
-        a.t0 = t0;
-        if (sk == 512 && a.K % 512 == 0) launch_mfma_lds<512, 1>(a, dual, st);  // two tiles would take 133 KB of LDS per block
-        else nt == 2 ? launch_mfma_lds<256, 2>(a, dual, st) : launch_mfma_lds<256, 1>(a, dual, st);
-        const int r = check_launch("matvec_mfma_lds");
-        if (r != SLHIP_OK) return r;
-    }
-    return SLHIP_OK;
+    a.t0 = 0;
+    if (sk == 512 && a.K % 512 == 0) launch_mfma_lds<512, 1>(a, dual, st);  // two tiles would take 133 KB of LDS per block
+    else nt == 2 ? launch_mfma_lds<256, 2>(a, dual, st) : launch_mfma_lds<256, 1>(a, dual, st);
+    return check_launch("matvec_mfma_lds");
 }
 
 // Tokens from which bf16 and f16 weights take the matrix cores (SLHIP_MATVEC_MFMA_MIN_T; 0 disables): below it the VALU
 // kernel is already at the HBM rate. Measured with bf16 weights at 14336 x 4096 (dual, us, VALU / matrix cores) at T = 2: f32
 // x 41.6 / 44.3, bf16 x 45.1 / 40.0; at T = 3: f32 x 51.5 / 43.6. From two tokens where the VALU kernel cannot hold both
-// tokens' x at once (K = 14336, N = 4096: bf16 49.1 / 23.5, f16 50.2 / 35.6). f16 weights take two bf16 parts: pairs with f32
-// x two tokens later while the VALU kernel holds four tokens' x (dual at [4096, 4096] and [14336, 4096]: T = 3 18.7 / 19.5,
-// 49.9 / 60.4; T = 5 38.0 / 19.4, 97.9 / 63.2; one matrix T = 3 12.0 / 12.8, 34.1 / 29.7).
+// tokens' x at once (K = 14336, N = 4096: bf16 49.1 / 23.5, f16 50.2 / 35.6). f16 weights take two bf16 parts, so a little
+// later while the VALU kernel holds four tokens' x (K up to 4096): two tokens with f32 x (one matrix of K = N = 4096 at T = 3
+// 13.1 / 14.9, T = 4 12.8 / 15.0, T = 5 25 / 15; pair T = 3 20 / 24, T = 5 39 / 22), one with bf16 x (pair of K = 2048,
+// N = 16384 at T = 2 26.8 / 33.0, T = 3 30.6 / 33.2; one matrix T = 2 15.3 / 18.4, T = 3 23 / 18), three for few rows (N = 1024,
+// T = 3 8.2 / 10.3, T = 5 16 / 10), and with f32 x while it holds eight (K = 2048, N = 1024: T = 8 7.5 / 8.7, pair 9.8 / 12.3).
 template <int WT>
-static int mfma_min_tokens(const MatvecArgs& a, bool dual)
+static int mfma_min_tokens(const MatvecArgs& a)
 {
-    const bool late = WT == SLHIP_F16 && dual && a.xt == SLHIP_F32 && token_tile(4, a.K) == 4;
+    const bool late = WT == SLHIP_F16 && token_tile(4, a.K) == 4;
     const int usual = a.xt == SLHIP_BF16 || token_tile(2, a.K) < 2 ? 2 : 3;
     const int mt = env_int("SLHIP_MATVEC_MFMA_MIN_T", usual);
-    return mt > 0 && late ? mt + 2 : mt;
+    if (mt <= 0 || !late) return mt;
+    if (a.xt == SLHIP_F32) return mt + (a.N > 2048 || token_tile(8, a.K) < 8 ? 2 : 6);
+    return mt + (a.N > 2048 ? 1 : 3);
 }
 
 // Whether a bf16 launch of up to 16 tokens is faster on the LDS-staged kernel above than on matvec_kw: where
 // matvec_kw's blocks no longer go round the chip once (it then pays whole further rounds). Measured at K = 4096 (us,
-// LDS-staged / matvec_kw at 3 tokens; 16): pairs, f32 x, N = 8192 25.6 / 24.7; 32.5 / 25.6, N = 14336 44.7 / 45.7;
-// 44.6 / 50.6; pairs, bf16 x, N = 4096 15.3 / 13.3; 15.7 / 13.8, N = 6144 18.4 / 19.0; 21.0 / 19.6, N = 14336 40.0 /
-// 43.9; 43.5 / 46.6; one matrix, bf16 x, N = 14336 21.2 / 19.7; 26.5 / 20.0, N = 20480 29.3 / 34.8; 36.8 / 38.8; one
-// matrix, f32 x, N = 20480 37.8 / 36.9; 45.3 / 43.4, N = 28672 45.7 / 47.2; 59.8 / 51.7.
+// LDS-staged / matvec_kw at 3 tokens; 8; 16): pairs, bf16 x, N = 4096 15.7 / 14.7; - ; 16.4 / 15.0, N = 7168 20.7 / 24.2; - ;
+// 22.8 / 25.0, N = 14336 39.3 / 43.4; - ; 41.0 / 46.0. f32 x, N = 7168 12 % faster; 5 %; 14 % slower, N = 10240 29 % faster;
+// 31 %; 1 %, N = 14336 6 % faster; 4 %; 8 %. One matrix, bf16 x, N = 8192 15 % faster; 13 %; 1 % slower (K = 2048 16 %, 16 %,
+// 19 % slower; K = 8192 10 %, 11 %, 13 % slower), N = 18432 36 % faster; 37 %; 23 %. One matrix with f32 x stays on matvec_kw,
+// whose sums are closer (a part of x at a time into the running sum rounds three times as often).
 static bool mfma_lds_better(const MatvecArgs& a, bool dual)
 {
     if (a.K % 256 != 0 || a.T > 16 || (a.T < 3 && a.xt == SLHIP_F32)) return false;
@@ -1249,7 +1250,7 @@ template <int WT>
 static int run_dense(MatvecArgs a, bool dual, hipStream_t st)
 {
     if constexpr (WT != SLHIP_F32) {
-        const int mt = mfma_min_tokens<WT>(a, dual);
+        const int mt = mfma_min_tokens<WT>(a);
         if (mt > 0 && a.K % 64 == 0 && a.T >= mt) {
             if (WT == SLHIP_BF16 && mfma_lds_better(a, dual)) return run_mfma(a, dual, st);
             const int r = run_kw(WT == SLHIP_BF16 ? SLHIP_FMT_BF16 : SLHIP_FMT_F16, a, dual, st);
