@@ -116,22 +116,52 @@ bool matvec_q8_fits(int fmt, int64_t K, bool dual)
 // counted. Q4_K, K = 4096, us here / there: N = 4096 8.4 / 13 (T = 4), 8.4 / 16 (T = 16), 10.4 / 28 (T = 31); N = 14336
 // 14.5 / 15.2, 14.9 / 20, 21.4 / 37; K = 14336, N = 4096 15 / 33, 16 / 42, 21 / 81; T = 2: 8.5 / 8.6; dual, N = 14336
 // (g = 1792) 23.6 / 25.8 (T = 16). Past the lines below: the same 23 / 21.9 (T = 4), 23 / 22.8 (T = 8); Q6_K, N = 14336
-// 21.8 / 16.7 (T = 3); Q8_0 dual, K = 2048, N = 8192 (g = 1024) 16.3 / 13.7 (T = 16); Q5_1, N = 128256 251 / 223 (T = 31).
+// 21.8 / 16.7 (T = 3). The lines lie by format, from sweeps at K = 2048 .. 8192, N = 2048 .. 40960, T = 3 .. 31; past them, K =
+// 4096: Q4_0 pair N = 14336 26.1 / 23.7 (T = 16), and again ahead N = 20480 31 / 35; IQ4_NL pair N = 14336 27.6 / 23.6 (T = 16);
+// IQ4_NL N = 14336 14.7 / 13.6 (T = 6), N = 32000 25.5 / 24.2 (T = 9), 26.3 / 29.2 (T = 16); Q4_1 N = 14336 16.5 / 13.6 (T = 8), pair
+// 55.8 / 42.0 (T = 17); Q5_0 N = 14336 18.8 / 16.4 (T = 8); Q5_1 17.6 / 15.8; Q8_0 pair N = 4096 12.2 / 11.1 (T = 8), N = 32768
+// 138 / 123 (T = 17); Q5_K pair N = 32768 137 / 122 (T = 17); Q6_K pair N = 13824, K = 5120 62.5 / 53 (T = 6), Q4_K pair N =
+// 8200, K = 3072 17.3 / 15.7 (T = 9), Q5_0 pair N = 8192, K = 1024 20.9 / 15.0 (T = 17).
 static int kw8_tiles(int fmt, const I8Args& a, bool dual)
 {
     const int env = i8_mfma_env();
     if (a.K % 256 != 0 || env == 0 || a.T < env || !matvec_q8_fits(fmt, a.K, dual)) return 0;
     const int64_t rows = (a.N + 15) / 16, g = dual ? 2 * rows : rows;
     const bool small = kw8_two_tiles(fmt);
+    // (the lines count the groups up by the idle share of the waves, where K has no whole number of stages for each)
+    const int64_t stages = a.K / 256, slots = (stages + 7) / 8 * 8, groups = g * slots / stages;
+    const bool even = slots == stages;
+    auto most = [&](int64_t one, int64_t pair) { return groups <= (dual ? pair : one); };
+    constexpr int64_t kAny = INT64_MAX;
     bool take;
-    if (a.T > 16)
-        take = g <= 2048 || (fmt != SLHIP_FMT_Q5_0 && fmt != SLHIP_FMT_Q5_1);
-    else if (small)
-        take = a.T >= (g <= 1024 ? 3 : 9);
-    else if (a.wrow % 16 != 0)  // (the other kernels' matrix-core forms want 16-byte rows)
-        take = a.T >= 5;
-    else
-        take = g <= (dual ? 512 : 1024) && a.T >= (a.K >= 8192 ? 4 : 5);
+    if (a.T > 16) {
+        switch (fmt) {
+        case SLHIP_FMT_Q4_1: take = even ? most(kAny, 768) : most(1300, 768); break;
+        case SLHIP_FMT_Q5_0: take = even ? most(2048, 1536) : most(1300, 1280); break;
+        case SLHIP_FMT_Q5_1: take = even ? most(2048, 1280) : most(1300, 1280); break;
+        case SLHIP_FMT_Q8_0: take = even ? most(kAny, a.K < 8192 ? 1280 : kAny) : most(2500, 1280); break;
+        case SLHIP_FMT_Q5_K: take = even ? most(kAny, 2304) : most(kAny, 1300); break;
+        case SLHIP_FMT_Q6_K: take = even ? most(kAny, 3584) : most(kAny, 1800); break;
+        case SLHIP_FMT_IQ4_NL: take = even || most(2500, 2500); break;
+        default: take = even || most(kAny, 4000);
+        }
+    } else if (small) {
+        take = a.T >= (g > 1024 ? 9 : fmt == SLHIP_FMT_Q4_0 ? 4 : 3);
+        if (dual && g > 1024) take = take && (a.K % 2048 == 0 || a.K > 8192);  // (else its eight waves' stages are uneven)
+        if (fmt == SLHIP_FMT_IQ4_NL) take = take && ((a.T > 12 && even) || most(512, 1536)) && most(kAny, 1536);
+        if (fmt == SLHIP_FMT_Q4_0) take = take && (g > 2048 || most(kAny, 1536));
+    } else if (a.wrow % 16 != 0) {  // (the other kernels' matrix-core forms want 16-byte rows)
+        take = a.T >= 5 && most(kAny, 1024);
+    } else {
+        take = a.T >= (a.K < 8192 || fmt == SLHIP_FMT_Q8_0 || fmt == SLHIP_FMT_Q6_K ? 5 : 4);
+        switch (fmt) {
+        case SLHIP_FMT_Q4_1:
+        case SLHIP_FMT_Q5_0:
+        case SLHIP_FMT_Q5_1: take = take && most(512, 512); break;
+        case SLHIP_FMT_Q8_0: take = take && most(512, 256); break;
+        default: take = take && most(1024, 512);
+        }
+    }
     if (!take) return 0;
     // two tiles a block where one each would be more than two blocks a CU: N = 14336, T = 16 15.1 / 17.7; N = 4096 9.7 / 8.4
     return small && !dual && rows * ((a.T + 15) / 16) > 512 ? 2 : 1;

@@ -23,10 +23,12 @@ SINGLE = [
     ("q4_k", "f32", 3, 14336, 33), ("q4_0", "f32", 3, 768, 1), ("q6_k", "f32", 4, 8192, 40), ("q8_0", "f32", 3, 8192, 40),
     ("iq4_nl", "bf16", 16, 256, 16401), ("q4_k", "f32", 100, 256, 8193), ("q5_1", "f32", 17, 256, 32785), ("q6_k", "f32", 5, 768, 16401),
 ]
+SINGLE += [*[(f, "f32", 17, 2048, 8209) for f in FORMATS]]  # many row tiles, an even split of the stages
 PAIRS = [
     *[(f, 16, 512, 33) for f in FORMATS],
     *[(f, 17, 256, 8209) for f in FORMATS],
     ("q4_k", 5, 256, 8209), ("q8_0", 16, 256, 4113), ("q6_k", 31, 2304, 16),
+    *[(f, 17, 2048, 4113) for f in FORMATS], ("q4_0", 9, 2048, 16401), ("iq4_nl", 9, 2048, 8209), ("q4_k", 9, 2048, 8209),
 ]
 
 
