@@ -157,14 +157,14 @@ SINGLE_CASES = [  # (fmt, x dtype, y dtype, T, K, N)
     ("q8_0", "bf16", "f32", 3, 1024, 33),
     ("q4_0", "f32", "f32", 2, 2048, 33),     # two tokens: the VALU kernel
     ("q8_0", "f32", "bf16", 17, 2048, 40),   # two token groups, the second of one token
-    ("q4_0", "f32", "f32", 5, 1536, 24),     # K not a whole number of 1024-value stages: the VALU kernel
+    ("q4_0", "f32", "f32", 5, 1536, 24),     # K not a whole number of 1024-value stages
     ("q4_0", "bf16", "f32", 1, 8192, 17),    # one token, a partial block of rows
     ("q4_0", "f32", "bf16", 1, 4096, 1),     # a single row
-    ("q4_k", "f32", "f32", 5, 1024, 33),     # Q4_K from five tokens on the matrix cores: one stage
+    ("q4_k", "f32", "f32", 5, 1024, 33),     # one stage
     ("q4_k", "bf16", "bf16", 16, 4096, 50),
     ("q4_k", "f32", "bf16", 17, 2048, 40),   # two token groups, the second of one token
-    ("q4_k", "f32", "f32", 4, 1280, 24),     # K not a whole number of 1024-value stages: the VALU kernel
-    ("q6_k", "f32", "f32", 5, 1024, 33),     # Q6_K from five tokens on the matrix cores: one 840-byte stage
+    ("q4_k", "f32", "f32", 4, 1280, 24),     # K not a whole number of 1024-value stages
+    ("q6_k", "f32", "f32", 5, 1024, 33),     # one 840-byte stage
     ("q6_k", "bf16", "bf16", 16, 4096, 50),
     ("q6_k", "f32", "bf16", 17, 3072, 40),   # two token groups, the second of one token; three stages
     ("q5_0", "f32", "f32", 6, 2048, 33),     # the other block formats on the matrix cores (Q5: qh bits)
@@ -172,7 +172,7 @@ SINGLE_CASES = [  # (fmt, x dtype, y dtype, T, K, N)
     ("q5_1", "f32", "bf16", 3, 3072, 24),
     ("q5_k", "f32", "f32", 16, 4096, 40),
     ("q5_k", "bf16", "bf16", 7, 1024, 17),
-    ("q2_k", "f32", "f32", 1, 4096, 40),     # Q2_K and Q3_K: the VALU kernel below five tokens
+    ("q2_k", "f32", "f32", 1, 4096, 40),     # Q2_K and Q3_K: the VALU kernel below three tokens
     ("q2_k", "bf16", "f32", 4, 2048, 24),
     ("q3_k", "f32", "bf16", 2, 3072, 33),    # rows of 1320 bytes: 8-byte staging loads
     ("q3_k", "bf16", "bf16", 3, 2048, 33),
@@ -180,7 +180,7 @@ SINGLE_CASES = [  # (fmt, x dtype, y dtype, T, K, N)
     ("q3_k", "f32", "f32", 17, 1024, 24),
     ("q2_k", "f32", "f32", 1, 1280, 33),     # rows of 420 bytes (not 16-byte multiples): 4-byte staging loads
     ("q2_k", "bf16", "bf16", 3, 512, 17),    # 168 bytes
-    ("q2_k", "f32", "f32", 6, 1280, 19),     # five tokens or more, K not a multiple of 1024: the VALU kernel
+    ("q2_k", "f32", "f32", 6, 1280, 19),     # K not a multiple of 1024
 ]
 
 
@@ -258,8 +258,8 @@ DUAL_CASES = [  # (act, fmt, x dtype, y dtype, T, K, N): FusionTests.SwiGluDualM
     ("gelu_erf", "f16", "f32", "f32", 4, 4096, 64),
     ("silu", "bf16", "bf16", "bf16", 1, 4096, 14336),  # the Llama-3-8B decode FFN (C3's model)
     ("silu", "bf16", "bf16", "f32", 2, 4096, 72),      # bf16 x at two tokens: the matrix cores
-    ("gelu_tanh", "bf16", "bf16", "bf16", 16, 1024, 40),  # bf16 x at 16 tokens: one tile per block
-    ("silu", "bf16", "f32", "f32", 13, 1024, 72),      # f32 x above 12 tokens: two tiles per block
+    ("gelu_tanh", "bf16", "bf16", "bf16", 16, 1024, 40),  # bf16 x at 16 tokens
+    ("silu", "bf16", "f32", "f32", 13, 1024, 72),      # f32 x above 12 tokens
     ("silu", "q8_0", "f32", "f32", 1, 1024, 96),
     ("silu", "q8_0", "f32", "f32", 9, 1024, 96),
     ("silu", "q4_0", "f32", "f32", 1, 4096, 14336),
@@ -283,7 +283,7 @@ DUAL_CASES = [  # (act, fmt, x dtype, y dtype, T, K, N): FusionTests.SwiGluDualM
     ("gelu_erf", "q6_k", "bf16", "f32", 3, 768, 33),
     ("silu", "q4_k", "f32", "f32", 16, 4096, 14336),  # batched Q4_K_M decode FFN on the matrix cores
     ("gelu_erf", "q4_k", "bf16", "bf16", 6, 1024, 72),
-    ("silu", "q4_k", "f32", "f32", 4, 1024, 40),       # four tokens: still the VALU kernel
+    ("silu", "q4_k", "f32", "f32", 4, 1024, 40),       # four tokens
     ("silu", "q6_k", "f32", "f32", 16, 4096, 14336),  # batched decode with Q6_K weights on the matrix cores
     ("gelu_tanh", "q6_k", "bf16", "f32", 8, 2048, 40),
     ("silu", "q5_k", "f32", "f32", 16, 4096, 14336),  # a Q5_K_M decode FFN at 16 tokens
@@ -356,12 +356,12 @@ def test_empty_shapes_are_noops(device):
 @pytest.mark.parametrize("dual,dx,T,K,N", [
     (False, "f32", 1, 1024, 48), (False, "f32", 4, 2048, 40), (True, "f32", 5, 4096, 64),
     (True, "bf16", 17, 1024, 33), (False, "bf16", 33, 256, 17),
-    (True, "f32", 9, 320, 40),  # K not a multiple of the 256-value stage: operands loaded directly
+    (True, "f32", 9, 320, 40),  # K not a multiple of 256
 ])
 def test_bf16_paths_agree_with_oracle(device, monkeypatch, min_t, dual, dx, T, K, N):
-    """bf16 weights take the MFMA kernels from SLHIP_MATVEC_MFMA_MIN_T tokens on; every kernel meets the same
-    bound whichever T it is forced onto (ragged token and row tiles, one and two 16-row tiles per block, the
-    LDS-staged kernel and, for K off its stage size, the directly loaded one)."""
+    """bf16 weights take the matrix cores from SLHIP_MATVEC_MFMA_MIN_T tokens on; matvec_kw and the VALU kernel meet the
+    same bound whichever T they are forced onto (ragged token and row tiles; the LDS-staged kernel of many rows:
+    test_gpu_matvec_many_rows)."""
     monkeypatch.setenv("SLHIP_MATVEC_MFMA_MIN_T", min_t)
     seed = _seed("paths", min_t, dual, dx, T, K, N)
     rg, Wg = _weights("bf16", N, K, seed, 1)
@@ -460,8 +460,8 @@ def test_q4k_one_token_wide_range_and_zero_rows(device):
 
 
 def test_q4k_several_tokens_wide_range_and_zero_rows(device):
-    """The several-token Q4_K kernel (bf16 codes on the matrix cores, f32 x as two bf16 parts, the minimum
-    applied as -m * sum(x) per sub-block on the VALU): x spanning 2^-20 .. 2^12 within a block, exact zeros and
+    """The several-token Q4_K kernel (bf16 codes on the matrix cores, f32 x as three bf16 parts, the minimum
+    applied as -m * sum(x) per sub-block): x spanning 2^-20 .. 2^12 within a block, exact zeros and
     an outlier stay within the f32 bound per token; rows whose codes and minima are all zero give exactly 0."""
     N, K, T = 40, 2048, 5
     raw, W = _weights("q4_k", N, K, 23, 1)
