@@ -274,8 +274,9 @@ static bool jit_streams(const EwgArgs& a)
 
 // The streaming kernel is for launches that the caches cannot hold anyway; memory-bound either way. Rows of 4096 f32, two
 // inputs, sum and norm stored, us plain / streaming: 33 MB 13.7 / 15.8, 67 MB 17.8 / 19.2, 134 MB 26.5 / 25.5, 201 MB 45.7 /
-// 35.9, 268 MB 58 / 49.6, 403 MB 90 / 75, 537 MB 108 / 91 to 103 (by process). Streaming the group's own outputs too loses (537 MB
-// 101), and so do two bodies in one kernel (105). The flat form is level everywhere.
+// 35.9, 268 MB 58 / 49.6, 403 MB 90 / 75, 537 MB 101.9 / 89 on buffers that rotate; on the same
+// buffers in every pass 107 / 105, where the caches serve the plain loads a part of the last pass. Streaming the group's own outputs
+// too loses (537 MB rotating 101), and so do two bodies in one kernel (105). The flat form is level everywhere.
 constexpr int64_t kJitStreamBytes = 144ll << 20;
 
 static bool jit_large(const EwgArgs& a)

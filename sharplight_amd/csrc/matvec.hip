@@ -623,7 +623,8 @@ __global__ __launch_bounds__(kMqThreads) void matvec_quant(MatvecArgs a)
 // bf16 weights at several tokens on the matrix cores: v_mfma_f32_16x16x32_bf16 multiplies a 16-row weight
 // tile (A: lane l holds row l % 16, eight K values of group l / 16) by 16 tokens of x (B: lane l holds token
 // l % 16, the same K values) into a 16 x 16 f32 tile (lane l: rows 4 (l / 16) + i, token l % 16). f32 x is
-// split into three bf16 parts h + m + l = x exactly (split3: f32 has 24 significant bits, bf16 8), so every product w * part is exact and the sums stay f32: the
+// split into three bf16 parts h + m + l = x exactly (split3: f32 has 24 significant bits, bf16 8), so every
+// product w * part is exact and the sums stay f32: the
 // result has the error of f32 accumulation, like the VALU kernel. bf16 x is one part. A block of 8 waves
 // takes a 16-row tile (pair); the waves split K; partial tiles meet in LDS.
 constexpr int kMmWaves = 8;

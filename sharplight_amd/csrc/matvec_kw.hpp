@@ -22,7 +22,7 @@
 // exact and the sums are f32, so the result is the f32 evaluation of sum(scale * code * x) + min terms in
 // another order: within f32 accumulation of those terms.
 //
-// What bounds it: instruction issue (the matrix cores are busy ~20% at 16 tokens, the vector unit ~50%), x's split
+// What bounds it: instruction issue (Q6_K K = 14336, N = 4096, T = 6: the vector unit is busy 79%, the matrix cores 16%), x's split
 // above all, which is why the wider blocks (more 16-row groups per split) win as soon as they still fill the chip; the
 // dispatch (matvec_kw.hip) picks the shape. Against the launch per 16 tokens that it replaces (the previous kernels,
 // barriers per stage), K = 4096, f32 x, us: Q4_K N = 4096 12.8 -> 12.5 (T = 16), 51 -> 16 (T = 64), 102 -> 25 (T = 128);
