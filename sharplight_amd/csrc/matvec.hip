@@ -731,7 +731,12 @@ __global__ __launch_bounds__(64 * kMmWaves) void matvec_mfma_lds(MatvecArgs a)
             for (int p = 0; p < (XF32 ? 3 : 1); p++) {
 #pragma unroll
                 for (int tt = 0; tt < NT; tt++) {
-                    ag[tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(Ag[q][tt]), as_bf16x8(B[q][p]), ag[tt], 0, 0, 0);
+                    // (one matrix with bf16 x: the products first, added by the vector unit, which rounds once: 1.4e-7 -> 1.0e-7 of
+                    // the exact result; the other forms have no registers for it)
+                    constexpr bool apart = !DUAL && !XF32;
+                    const f32x4_t z = {0.0f, 0.0f, 0.0f, 0.0f};
+                    const f32x4_t d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(Ag[q][tt]), as_bf16x8(B[q][p]), apart ? z : ag[tt], 0, 0, 0);
+                    ag[tt] = apart ? ag[tt] + d : d;
                     if (DUAL)
                         au[tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(Au[q][tt]), as_bf16x8(B[q][p]), au[tt], 0, 0, 0);
                 }
