@@ -1368,7 +1368,7 @@ static int quant_ch(const MatvecArgs& a, int ch, hipStream_t st)
 template <int FMT, bool DUAL>
 static int quant_tt(const MatvecArgs& a, int tt, int ch, hipStream_t st)
 {
-    return tt == 1 ? quant_ch<FMT, 1, DUAL>(a, ch, st) : tt == 2 ? quant_ch<FMT, 2, DUAL>(a, ch, st) : quant_ch<FMT, 4, DUAL>(a, ch, st);
+    return tt == 1 ? quant_ch<FMT, 1, DUAL>(a, ch, st) : quant_ch<FMT, 2, DUAL>(a, ch, st);
 }
 
 template <int FMT, bool DUAL>
@@ -1420,11 +1420,7 @@ static int run_quant(MatvecArgs a, bool dual, hipStream_t st)
     constexpr int64_t kLongK = FMT == SLHIP_FMT_Q8_0 || FMT == SLHIP_FMT_Q6_K ? 512 : 1024;
     const int dflt = !long_row && quant_lds(2, a.K, a.wrow, dual) > kMaxLds ? 2 : 3;
     const int mt = env_int(Fmt<FMT>::K ? "SLHIP_MATVEC_KQ_MIN_T" : "SLHIP_MATVEC_MQ_MIN_T", dflt);
-    // Few rows at three and four tokens: one pass of four on the VALU kernel where K is off matvec_mq2's stages and so an
-    // uneven split for matvec_kw, too (K = 2560, N = 1024, T = 3, us, matvec_kw / VALU: Q4_0 9.6 / 7.0, pair 12.0 / 7.9; Q4_K
-    // 8.7 / 7.0; Q5_0 pair 14.5 / 8.6; N = 2048 pair 12.8 / 10.0; N = 4096 level).
-    const bool four = a.K % kLongK != 0 && a.N <= 2048 && a.T <= 4 && quant_lds(4, a.K, a.wrow, dual) <= kMaxLds;
-    if (mt > 0 && a.T >= mt && !(four && a.T > 2) && (!long_row || a.K % kLongK == 0)) {
+    if (mt > 0 && a.T >= mt && (!long_row || a.K % kLongK == 0)) {
         if (mq2_better(FMT, a, dual)) {
             const int r = run_mq2_any(FMT, a, dual, st);
             if (r != SLHIP_ERR_UNSUPPORTED) return r;
@@ -1438,7 +1434,7 @@ static int run_quant(MatvecArgs a, bool dual, hipStream_t st)
             env_int("SLHIP_KQ_MFMA", 1))
             return dual ? launch_kq_tile<FMT, true>(a, st) : launch_kq_tile<FMT, false>(a, st);
     }
-    const int tt = four && a.T > 2 ? 4 : a.T > 1 && quant_lds(2, a.K, a.wrow, dual) <= kMaxLds ? 2 : 1;
+    const int tt = a.T > 1 && quant_lds(2, a.K, a.wrow, dual) <= kMaxLds ? 2 : 1;
     if (long_row)
         return fail(SLHIP_ERR_UNSUPPORTED, "matvec: K = %lld does not fit in LDS for this format", static_cast<long long>(a.K));
     const int64_t per_lane = ((dual ? 2 : 1) * (a.wrow / 16) + 63) / 64;

@@ -56,13 +56,6 @@ def test_few_stages(device, fmt, dx, T, K, N, pair):
     (check_pair if pair else check_product)(device, fmt, dx, T, K, N)
 
 
-@pytest.mark.parametrize("fmt", MQ)
-@pytest.mark.parametrize("dx,T,K,N,pair", [("f32", 3, 1280, 2047, False), ("bf16", 4, 2304, 40, True)])
-def test_four_tokens_of_few_rows(device, fmt, dx, T, K, N, pair):
-    """One pass of four tokens on the VALU kernel: K off the stages of matvec_mq2."""
-    (check_pair if pair else check_product)(device, fmt, dx, T, K, N)
-
-
 @pytest.mark.parametrize("fmt,dx,T,K,N", [
     ("q4_k", "f32", 19, 256, 40), ("q6_k", "f32", 19, 512, 40), ("q8_0", "bf16", 19, 512, 40), ("q2_k", "f32", 33, 256, 2900),  # matvec_kw
     ("q3_k", "f32", 19, 256, 40), ("q5_1", "f32", 50, 256, 2900),
