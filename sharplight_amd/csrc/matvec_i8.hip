@@ -116,12 +116,13 @@ bool matvec_q8_fits(int fmt, int64_t K, bool dual)
 // counted. Q4_K, K = 4096, us here / there: N = 4096 8.4 / 13 (T = 4), 8.4 / 16 (T = 16), 10.4 / 28 (T = 31); N = 14336
 // 14.5 / 15.2, 14.9 / 20, 21.4 / 37; K = 14336, N = 4096 15 / 33, 16 / 42, 21 / 81; T = 2: 8.5 / 8.6; dual, N = 14336
 // (g = 1792) 23.6 / 25.8 (T = 16). Past the lines below: the same 23 / 21.9 (T = 4), 23 / 22.8 (T = 8); Q6_K, N = 14336
-// 21.8 / 16.7 (T = 3). The lines lie by format, from sweeps at K = 2048 .. 8192, N = 2048 .. 40960, T = 3 .. 31; past them, K =
-// 4096: Q4_0 pair N = 14336 26.1 / 23.7 (T = 16), and again ahead N = 20480 31 / 35; IQ4_NL pair N = 14336 27.6 / 23.6 (T = 16);
-// IQ4_NL N = 14336 14.7 / 13.6 (T = 6), N = 32000 25.5 / 24.2 (T = 9), 26.3 / 29.2 (T = 16); Q4_1 N = 14336 16.5 / 13.6 (T = 8), pair
-// 55.8 / 42.0 (T = 17); Q5_0 N = 14336 18.8 / 16.4 (T = 8); Q5_1 17.6 / 15.8; Q8_0 pair N = 4096 12.2 / 11.1 (T = 8), N = 32768
-// 138 / 123 (T = 17); Q5_K pair N = 32768 137 / 122 (T = 17); Q6_K pair N = 13824, K = 5120 62.5 / 53 (T = 6), Q4_K pair N =
-// 8200, K = 3072 17.3 / 15.7 (T = 9), Q5_0 pair N = 8192, K = 1024 20.9 / 15.0 (T = 17).
+// 21.8 / 16.7 (T = 3). The lines lie by format, from sweeps at K = 512 .. 8192, N = 2048 .. 40960, T = 3 .. 31; past them, K
+// = 4096: IQ4_NL pair N = 14336 27.6 / 23.6 (T = 16); IQ4_NL N = 14336 14.7 / 13.6 (T = 6), N = 32000 25.5 / 24.2 (T = 9),
+// 26.3 / 29.2 (T = 16); Q4_1 N = 14336 16.5 / 13.6 (T = 8), pair 55.8 / 42.0 (T = 17); Q5_1 N = 14336 17.6 / 15.8 (T = 8);
+// Q8_0 pair N = 4096 12.2 / 11.1 (T = 8), N = 32768 138 / 123 (T = 17); Q5_K pair N = 32768 137 / 122 (T = 17); Q4_K pair N
+// = 8200, K = 3072 17.3 / 15.7 (T = 9). Q4_0, Q5_0 and Q6_K keep further lines, though Q4_0 pair N = 14336 takes 26.1 / 23.7
+// (T = 16) and Q5_0 N = 14336 18.8 / 16.4 (T = 8): their codes are signed here, while the other kernels subtract an offset
+// term and are further from the exact result (Q4_0 pair 1.5e-7 / 2.8e-7, Q5_0 9.8e-8 / 2.3e-7, Q6_K pair 1.5e-7 / 1.9e-7).
 static int kw8_tiles(int fmt, const I8Args& a, bool dual)
 {
     const int env = i8_mfma_env();
@@ -133,33 +134,32 @@ static int kw8_tiles(int fmt, const I8Args& a, bool dual)
     const bool even = slots == stages;
     auto most = [&](int64_t one, int64_t pair) { return groups <= (dual ? pair : one); };
     constexpr int64_t kAny = INT64_MAX;
+    const bool offset = fmt == SLHIP_FMT_Q4_0 || fmt == SLHIP_FMT_Q5_0 || fmt == SLHIP_FMT_Q6_K;
     bool take;
-    if (a.T > 16) {
+    if (offset && a.T > 16) {
+        take = fmt != SLHIP_FMT_Q5_0 || g <= 2048;
+    } else if (a.T > 16) {
         switch (fmt) {
         case SLHIP_FMT_Q4_1: take = even ? most(kAny, 768) : most(1300, 768); break;
-        case SLHIP_FMT_Q5_0: take = even ? most(2048, 1536) : most(1300, 1280); break;
         case SLHIP_FMT_Q5_1: take = even ? most(2048, 1280) : most(1300, 1280); break;
         case SLHIP_FMT_Q8_0: take = even ? most(kAny, a.K < 8192 ? 1280 : kAny) : most(2500, 1280); break;
         case SLHIP_FMT_Q5_K: take = even ? most(kAny, 2304) : most(kAny, 1300); break;
-        case SLHIP_FMT_Q6_K: take = even ? most(kAny, 3584) : most(kAny, 1800); break;
         case SLHIP_FMT_IQ4_NL: take = even || most(2500, 2500); break;
         default: take = even || most(kAny, 4000);
         }
     } else if (small) {
-        take = a.T >= (g > 1024 ? 9 : fmt == SLHIP_FMT_Q4_0 ? 4 : 3);
-        if (dual && g > 1024) take = take && (a.K % 2048 == 0 || a.K > 8192);  // (else its eight waves' stages are uneven)
+        take = a.T >= (g > 1024 ? 9 : 3);
+        if (dual && g > 1024 && !offset) take = take && (a.K % 2048 == 0 || a.K > 8192);  // (else its eight waves' stages are uneven)
         if (fmt == SLHIP_FMT_IQ4_NL) take = take && ((a.T > 12 && even) || most(512, 1536)) && most(kAny, 1536);
-        if (fmt == SLHIP_FMT_Q4_0) take = take && (g > 2048 || most(kAny, 1536));
     } else if (a.wrow % 16 != 0) {  // (the other kernels' matrix-core forms want 16-byte rows)
-        take = a.T >= 5 && most(kAny, 1024);
+        take = a.T >= 5;
     } else {
-        take = a.T >= (a.K < 8192 || fmt == SLHIP_FMT_Q8_0 || fmt == SLHIP_FMT_Q6_K ? 5 : 4);
+        take = a.T >= (a.K < 8192 || fmt == SLHIP_FMT_Q8_0 ? 5 : 4);
         switch (fmt) {
         case SLHIP_FMT_Q4_1:
-        case SLHIP_FMT_Q5_0:
         case SLHIP_FMT_Q5_1: take = take && most(512, 512); break;
         case SLHIP_FMT_Q8_0: take = take && most(512, 256); break;
-        default: take = take && most(1024, 512);
+        default: take = take && g <= (dual ? 512 : 1024);
         }
     }
     if (!take) return 0;
